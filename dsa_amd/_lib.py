@@ -81,6 +81,11 @@ SIGNATURES = {
     "dsa_indexer_topk_ws": (_i32, [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _vp, _i64, _vp]),
 }
 
+# Entry points of csrc/host_entry.h, called by this package only.
+PRIVATE_SIGNATURES = {
+    "dsa_kv_quantize_rows": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp]),
+}
+
 _lock = threading.Lock()
 _lib = None
 
@@ -95,7 +100,7 @@ def load() -> ctypes.CDLL:
                     f"{LIB_PATH} is missing: build it with `python -m dsa_amd.build` "
                     "(dsa_amd has no CPU or fallback path)")
             lib = ctypes.CDLL(str(LIB_PATH))
-            for name, (res, args) in SIGNATURES.items():
+            for name, (res, args) in {**SIGNATURES, **PRIVATE_SIGNATURES}.items():
                 fn = getattr(lib, name)
                 fn.restype = res
                 fn.argtypes = args

@@ -14,12 +14,16 @@ instruction per two values.  :func:`quantize_kv_fp8` writes such rows from a
 bf16 cache: per 128-dim block the scale is the smallest power of two with
 ``amax / scale <= 448`` (e4m3 is floating point, so a power-of-two scale
 costs no relative precision), or exactly ``amax / 448`` with
-``pow2_scales=False``.  It is ordinary tensor code (the cache writer sits
-outside the attention's hot path).
+``pow2_scales=False``.  Tensors on a ROCm GPU are written by one kernel
+(``csrc/kv_rows.hip``), any other call (CPU tensors, traced or transformed
+ones) by the same arithmetic as tensor code, to the same bytes.
 """
 from __future__ import annotations
 
 import torch
+
+from . import _lib
+from .api import _on_device
 
 FP8_ROW = 656
 E4M3_MAX = 448.0
@@ -33,6 +37,8 @@ def quantize_kv_fp8(kv, k_rope, pow2_scales: bool = True):
     if kv.dtype != torch.bfloat16 or k_rope.dtype != torch.bfloat16:
         raise ValueError("kv and k_rope must be bfloat16")
     lead = kv.shape[:-1]
+    if _plain_gpu_pair(kv, k_rope):
+        return _quantize_gpu(kv.contiguous(), k_rope.contiguous(), lead, pow2_scales)
     x = kv.float().reshape(*lead, 4, 128)
     amax = x.abs().amax(-1, keepdim=True)
     scale = torch.where(amax > 0, amax / E4M3_MAX, torch.ones_like(amax))
@@ -44,3 +50,27 @@ def quantize_kv_fp8(kv, k_rope, pow2_scales: bool = True):
                       scale.reshape(*lead, 4).contiguous().view(torch.uint8),
                       k_rope.contiguous().view(torch.uint8)], dim=-1)
     return rows.contiguous()
+
+
+def _plain_gpu_pair(kv, k_rope):
+    """Whether the kernel may read these two tensors: ordinary eager tensors
+    of one ROCm GPU (no subclass, tracing, dispatch mode or functorch level
+    between the caller and the storage) with at least one row."""
+    return (type(kv) is torch.Tensor and type(k_rope) is torch.Tensor and kv.is_cuda and kv.device == k_rope.device
+            and torch.version.hip is not None and kv.numel() > 0 and not torch.compiler.is_compiling()
+            and not torch.jit.is_tracing() and not torch._C._are_functorch_transforms_active()
+            and torch._C._len_torch_dispatch_stack() == 0 and not (kv.is_neg() or k_rope.is_neg()))
+
+
+def _quantize_gpu(kv, k_rope, lead, pow2_scales):
+    device = kv.device
+    # a view may start anywhere in its storage: the kernel's loads are 16 and 4 bytes wide
+    kv = kv.clone() if kv.data_ptr() % 16 else kv
+    k_rope = k_rope.clone() if k_rope.data_ptr() % 4 else k_rope
+    rows = torch.empty((*lead, FP8_ROW), device=device, dtype=torch.uint8)
+    with _on_device(device):
+        rc = _lib.load().dsa_kv_quantize_rows(kv.data_ptr(), k_rope.data_ptr(), rows.data_ptr(), kv.numel() // 512,
+                                              1 if pow2_scales else 0,
+                                              torch._C._cuda_getCurrentRawStream(device.index))
+    _lib.check(rc, "dsa_kv_quantize_rows")
+    return rows
