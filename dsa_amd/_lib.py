@@ -84,6 +84,8 @@ SIGNATURES = {
 # Entry points of csrc/host_entry.h, called by this package only.
 PRIVATE_SIGNATURES = {
     "dsa_kv_quantize_rows": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp]),
+    "dsa_kv_expand_rows": (_i32, [_vp, _vp, _vp, _i32, _i32, _vp, _i32, _i32, _i32, _vp]),
+    "dsa_bucket_indices_paged": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _vp, _i32, _i32, _i32, _vp]),
 }
 
 _lock = threading.Lock()

@@ -157,6 +157,30 @@ def buckets_rows(shape) -> bool:
     return shape[0] * shape[1] >= BUCKET_MIN_TOKENS and shape[4] <= BUCKET_MAX_TOPK
 
 
+# Gathers per cache row from which an fp8 call expands its cache first.  The
+# narrow kernels expand every gathered slot in LDS, once per head group: with
+# one group (16, 32 or 64 heads) the pass over the cache pays from about 10
+# gathers a row (16 heads, 300 x 2048 of 65536 rows, 9.4 gathers: 125 against
+# 137 us; 256 x 2048, 8 gathers: 87 against 77 us), with more groups from
+# below 4 (128 heads, 256 x 1024 of 65536 rows: 91 against 128 us).
+EXPAND_MIN_REUSE, EXPAND_MIN_REUSE_GROUPS = 12, 4
+EXPAND_MAX_BYTES = 1 << 30  # largest expanded cache (1,152 bytes a row)
+
+
+def expands_rows(shape) -> bool:
+    """Whether a default-plan call on fp8 rows first expands its whole cache to
+    bf16 rows (kv_rows.hip) and then runs as a bf16 call: prefill-sized calls
+    that gather every row of the logical ``[B, L]`` cache many times, where
+    one pass over the cache costs less than expanding each gathered slot and
+    the faster bf16 kernels apply (128 heads, 2048 queries of 32768 rows: 986
+    against 1,780 us)."""
+    batch, queries, heads, length, topk = shape
+    rows = batch * length
+    reuse = EXPAND_MIN_REUSE if heads in (16, 32, 64) else EXPAND_MIN_REUSE_GROUPS
+    return (buckets_rows(shape) and batch * queries * topk >= reuse * rows
+            and rows * 2 * (HEAD_DIM + ROPE_DIM) <= EXPAND_MAX_BYTES)
+
+
 def bucket_lds_bytes(topk: int) -> int:
     """LDS of the bucketing kernel: 65 counts per 64-slot chunk, 65 bucket
     bases and the assembled row, 4 bytes each."""
@@ -340,7 +364,10 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
     slot whose block entry is outside ``[0, num_blocks)`` is masked.  An fp8
     kv cache is a uint8 ``kv [B, L, 1, 656]`` (or pool) of rows written by
     :func:`dsa_amd.quantize_kv_fp8`, with ``k_rope=None``; the kernel computes
-    with ``bf16(fp32(e4m3) * scale)`` latent values.
+    with ``bf16(fp32(e4m3) * scale)`` latent values.  A prefill-sized call
+    without a ``config`` that gathers each cache row often (:func:`expands_rows`)
+    first writes those values into a buffer of its own and then runs as a bf16
+    call: the same values through other kernels.
 
     ``w_uv`` (bf16 ``[H, dv, 512]``, dv a multiple of 64 up to 256; heads may
     be any stride apart, so ``wkv_b.view(H, d_nope + dv, 512)[:, -dv:]`` goes
@@ -377,10 +404,16 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
     if cores is None:
         cores = _device_cus(device)
     default_plan = config is None
-    config, partials, launches, plan, fused, groups = _call_plan(shape, config, cores, fp8,
-                                                                 None if uv is None else uv[0])
+    uv_dim = None if uv is None else uv[0]
+    config, partials, launches, plan, fused, groups = _call_plan(shape, config, cores, fp8, uv_dim)
     if fused and arrivals is not None and arrivals.numel() < groups:
         raise ValueError(f"arrivals holds {arrivals.numel()} counters; this call needs {groups}")
+    expanded = None
+    if fp8 and default_plan and arrivals is None and expands_rows(shape):
+        expanded = _expanded_cache(kv, block_table, shape)
+        if expanded is not None:
+            config, partials, launches, plan, fused, groups = _call_plan(shape, None, cores, False, uv_dim)
+            launches = (Launch("expand_rows", _expand_grid(batch * length), 256, 0),) + launches
     bucket = buckets_rows(shape)
     if (default_plan and cores == _device_cus(device) and not fused and not fp8 and scale is None
             and block_table is None and uv is None and not bucket):
@@ -402,14 +435,31 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
     stream = torch._C._cuda_getCurrentRawStream(device.index)
     lib = _lib.load()
     idx_ptr = indices.data_ptr()
+    kv_ptr, rope_ptr = kv.data_ptr(), None if k_rope is None else k_rope.data_ptr()
+    if expanded is not None:
+        pages = (None, 0, 0, 0) if block_table is None else (block_table.data_ptr(), block_table.shape[1],
+                                                             kv.shape[1], kv.shape[0])
+        rope_row = batch * length * 2 * HEAD_DIM  # the rope rows follow the latent ones
+        with _on_device(device):
+            rc = lib.dsa_kv_expand_rows(kv_ptr, expanded.data_ptr(), expanded.data_ptr() + rope_row, batch, length,
+                                        *pages, stream)
+        if rc:
+            _lib.check(rc, "dsa_kv_expand_rows")
+        kv_ptr, rope_ptr = expanded.data_ptr(), expanded.data_ptr() + rope_row
     if bucket:
         order = torch.empty_like(indices)
         with _on_device(device):
-            rc = lib.dsa_bucket_indices(idx_ptr, order.data_ptr(), batch * queries, topk, length, stream)
+            if expanded is not None and block_table is not None:
+                rc = lib.dsa_bucket_indices_paged(idx_ptr, order.data_ptr(), batch, queries, topk, length, *pages,
+                                                  stream)
+            else:
+                rc = lib.dsa_bucket_indices(idx_ptr, order.data_ptr(), batch * queries, topk, length, stream)
         if rc:
             _lib.check(rc, "dsa_bucket_indices")
         idx_ptr = order.data_ptr()
-    args = (q.data_ptr(), kv.data_ptr(), q_rope.data_ptr(), None if k_rope is None else k_rope.data_ptr(),
+    if expanded is not None:  # from here on a contiguous bf16 call
+        fp8, block_table = False, None
+    args = (q.data_ptr(), kv_ptr, q_rope.data_ptr(), rope_ptr,
             idx_ptr, output.data_ptr(), maximum.data_ptr(), denominator.data_ptr(),
             part_o, part_m, part_l, batch, queries, heads, length, topk)
     merge_uv = uv is not None and config.split > 1
@@ -444,6 +494,22 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
     if return_kernels:
         return result, launches
     return result
+
+
+def _expanded_cache(kv, block_table, shape):
+    """Buffer of the bf16 rows of an fp8 call's logical cache, latent rows then
+    rope rows; None where the pool is beyond what a call accepts (the call
+    itself then says so) or the memory is not there (it runs on the fp8 rows)."""
+    if block_table is not None and kv.shape[0] * kv.shape[1] >= 1 << 25:
+        return None
+    try:
+        return torch.empty(shape[0] * shape[3] * (HEAD_DIM + ROPE_DIM), device=kv.device, dtype=torch.bfloat16)
+    except torch.OutOfMemoryError:
+        return None
+
+
+def _expand_grid(rows: int) -> int:
+    return min(-(-rows // 16), 4096)
 
 
 def _options(scale, fp8, kv, block_table):

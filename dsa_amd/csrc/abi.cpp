@@ -13,6 +13,7 @@
 #include <cstring>
 
 #include "../../include/dsa_mi355x.h"
+#include "host_entry.h"
 #include "kernels.h"
 
 namespace {
@@ -237,19 +238,39 @@ int dsa_merge(const float* part_o, const float* part_m, const float* part_l, uin
     return 0;
 }
 
-int dsa_bucket_indices(const int32_t* idx, int32_t* out, int tokens, int TOPK, int L, void* stream_) {
-    const hipStream_t stream = static_cast<hipStream_t>(stream_);
+namespace {
+
+int bucket_impl(const int32_t* idx, int32_t* out, int64_t tokens, int TOPK, int L, const dsa::BlockTable& bt,
+                hipStream_t stream) {
     if (!idx || !out) return fail(-1, "NULL pointer argument");
     if (tokens <= 0 || TOPK <= 0 || L <= 0)
-        return fail(-1, "tokens, TOPK and L must be positive (got %d, %d, %d)", tokens, TOPK, L);
+        return fail(-1, "tokens, TOPK and L must be positive (got %lld, %d, %d)", (long long)tokens, TOPK, L);
     if (TOPK > dsa::kBucketMaxTopk)
         return fail(-1, "TOPK must be at most %d here (got %d)", dsa::kBucketMaxTopk, TOPK);
     if (idx == out) return fail(-1, "out must not alias idx");
     if (((uintptr_t)idx | (uintptr_t)out) & 3) return fail(-1, "idx and out must be 4-byte aligned");
-    const int rc = dsa::launch_bucket_rows(idx, out, tokens, TOPK, L, stream);
+    const int rc = dsa::launch_bucket_rows(idx, out, tokens, TOPK, L, bt, stream);
     if (rc) return hip_fail(rc, "bucket launch");
     g_err[0] = 0;
     return 0;
+}
+
+}  // namespace
+
+int dsa_bucket_indices(const int32_t* idx, int32_t* out, int tokens, int TOPK, int L, void* stream) {
+    return bucket_impl(idx, out, tokens, TOPK, L, dsa::BlockTable{}, static_cast<hipStream_t>(stream));
+}
+
+int dsa_bucket_indices_paged(const int32_t* idx, int32_t* out, int B, int SQ, int TOPK, int L,
+                             const int32_t* block_table, int max_blocks, int block_size, int num_blocks,
+                             void* stream) {
+    if (B <= 0 || SQ <= 0 || (int64_t)B * SQ > INT32_MAX) return fail(-1, "B and SQ must be positive, B * SQ int32");
+    if (!block_table || ((uintptr_t)block_table & 3)) return fail(-1, "block_table must be non-NULL, 4-byte aligned");
+    if (max_blocks <= 0 || block_size <= 0 || num_blocks <= 0 || (int64_t)max_blocks * block_size != L)
+        return fail(-1, "L must equal max_blocks * block_size, num_blocks be positive");
+    return bucket_impl(idx, out, (int64_t)B * SQ, TOPK, L,
+                       dsa::BlockTable{block_table, max_blocks, block_size, num_blocks, SQ},
+                       static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

@@ -41,7 +41,7 @@ __device__ inline uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p
 template <int NR>
 __global__ __launch_bounds__(kThreads) void bucket_rows_kernel(const int32_t* __restrict__ idx,
                                                                int32_t* __restrict__ out, int topk, uint32_t kv_len,
-                                                               int shift) {
+                                                               int shift, BlockTable bt) {
     // LDS: counts[chunk][bucket] (then each bucket's offsets within it), the
     // buckets' bases, the assembled row
     extern __shared__ int32_t lds[];
@@ -58,6 +58,16 @@ __global__ __launch_bounds__(kThreads) void bucket_rows_kernel(const int32_t* __
 #pragma unroll
     for (int r = 0; r < NR; ++r) val[r] = src[min(((wave + 4 * r) << 6) + lane, topk - 1)];
     for (int i = tid; i < chunks * kBuckets; i += kThreads) counts[i] = 0;
+    if (bt.table != nullptr) {  // uniform: slots behind unbacked blocks are masked here
+        const int32_t* entries = bt.table + row / bt.queries * bt.max_blocks;
+        int blk[NR];
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+            blk[r] = entries[(uint32_t)val[r] < kv_len ? (uint32_t)val[r] / (uint32_t)bt.block_size : 0u];
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+            if ((uint32_t)blk[r] >= (uint32_t)bt.num_blocks) val[r] = -1;
+    }
     __syncthreads();
 
     // Each slot's bucket and its rank among the chunk's slots of that bucket
@@ -149,21 +159,22 @@ size_t bucket_rows_lds_bytes(int topk) {
     return sizeof(int32_t) * ((size_t)((topk + 63) / 64) * kBuckets + kBuckets + topk);
 }
 
-int launch_bucket_rows(const int32_t* idx, int32_t* out, int64_t tokens, int topk, int kv_len, hipStream_t stream) {
+int launch_bucket_rows(const int32_t* idx, int32_t* out, int64_t tokens, int topk, int kv_len, const BlockTable& bt,
+                       hipStream_t stream) {
     const dim3 grid((unsigned)tokens), block(kThreads);
     const size_t lds = bucket_rows_lds_bytes(topk);
     const uint32_t len = (uint32_t)kv_len;
     const int shift = bucket_shift(kv_len);
     if (topk <= 256)
-        hipLaunchKernelGGL(bucket_rows_kernel<1>, grid, block, lds, stream, idx, out, topk, len, shift);
+        hipLaunchKernelGGL(bucket_rows_kernel<1>, grid, block, lds, stream, idx, out, topk, len, shift, bt);
     else if (topk <= 512)
-        hipLaunchKernelGGL(bucket_rows_kernel<2>, grid, block, lds, stream, idx, out, topk, len, shift);
+        hipLaunchKernelGGL(bucket_rows_kernel<2>, grid, block, lds, stream, idx, out, topk, len, shift, bt);
     else if (topk <= 1024)
-        hipLaunchKernelGGL(bucket_rows_kernel<4>, grid, block, lds, stream, idx, out, topk, len, shift);
+        hipLaunchKernelGGL(bucket_rows_kernel<4>, grid, block, lds, stream, idx, out, topk, len, shift, bt);
     else if (topk <= 2048)
-        hipLaunchKernelGGL(bucket_rows_kernel<8>, grid, block, lds, stream, idx, out, topk, len, shift);
+        hipLaunchKernelGGL(bucket_rows_kernel<8>, grid, block, lds, stream, idx, out, topk, len, shift, bt);
     else
-        hipLaunchKernelGGL(bucket_rows_kernel<16>, grid, block, lds, stream, idx, out, topk, len, shift);
+        hipLaunchKernelGGL(bucket_rows_kernel<16>, grid, block, lds, stream, idx, out, topk, len, shift, bt);
     return (int)hipGetLastError();
 }
 

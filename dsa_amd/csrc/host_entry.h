@@ -17,6 +17,20 @@ extern "C" {
 int dsa_kv_quantize_rows(const uint16_t* kv, const uint16_t* k_rope, uint8_t* out, int64_t rows, int pow2,
                          void* stream);
 
+// The bf16 rows of an fp8 cache: in [B * L, 656] or, with a block table (int32
+// [B, max_blocks], L = max_blocks * block_size), a pool of num_blocks *
+// block_size rows; kv [B * L, 512] (16-byte aligned), k_rope [B * L, 64].
+// Rows behind an entry outside [0, num_blocks) become zeros.
+int dsa_kv_expand_rows(const uint8_t* in, uint16_t* kv, uint16_t* k_rope, int B, int L, const int32_t* block_table,
+                       int max_blocks, int block_size, int num_blocks, void* stream);
+
+// dsa_bucket_indices for a paged cache whose rows are about to be addressed
+// without the block table: the same partition of idx [B * SQ, TOPK], with
+// every slot whose block entry lies outside [0, num_blocks) masked (-1).
+int dsa_bucket_indices_paged(const int32_t* idx, int32_t* out, int B, int SQ, int TOPK, int L,
+                             const int32_t* block_table, int max_blocks, int block_size, int num_blocks,
+                             void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -86,14 +86,24 @@ int64_t fwd_grid(const FwdParams& p);
 int launch_fwd(const FwdParams& p, int heads_per_group, int kv_waves, int tile_rows,
                int stages, int mfma, int pv_cols, hipStream_t stream);
 
+// A paged cache's block table (table NULL: contiguous rows), for the kernels
+// that run before the attention.  `queries`: rows of the index tensor that
+// share one table row (the query length).
+struct BlockTable {
+    const int32_t* table;
+    int max_blocks, block_size, num_blocks, queries;
+};
+
 // Largest TOPK the row bucketing handles (its LDS holds one row).
 constexpr int kBucketMaxTopk = 4096;
 
 // Enqueue the row bucketing of `tokens` index rows of `topk` entries: each
 // row stably partitioned by x >> bucket_shift(kv_len) for 0 <= x < kv_len,
 // every other entry last; returns a hipError_t.  topk in [1, kBucketMaxTopk],
-// kv_len >= 1; out may not alias idx.
-int launch_bucket_rows(const int32_t* idx, int32_t* out, int64_t tokens, int topk, int kv_len, hipStream_t stream);
+// kv_len >= 1; out may not alias idx.  With a block table, a slot whose block
+// entry lies outside the pool becomes -1 (and goes last).
+int launch_bucket_rows(const int32_t* idx, int32_t* out, int64_t tokens, int topk, int kv_len, const BlockTable& bt,
+                       hipStream_t stream);
 
 // The least shift with (kv_len - 1) >> shift < 64.
 int bucket_shift(int kv_len);

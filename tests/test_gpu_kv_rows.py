@@ -81,3 +81,70 @@ def test_empty_and_mixed_devices():
     assert dsa_amd.quantize_kv_fp8(kv.cuda(), kr.cuda()).shape == (0, 656)
     with pytest.raises(RuntimeError):
         dsa_amd.quantize_kv_fp8(torch.zeros(2, 512).bfloat16().cuda(), torch.zeros(2, 64).bfloat16())
+
+
+# ------------------------------------------------- the cache expanded to bf16
+
+def _expanding_case(batch, queries, heads, length, topk, block, seed):
+    """A call that expands its cache; returns (args, block table, contiguous
+    rows, the slots' validity through the table)."""
+    g = torch.Generator().manual_seed(seed)
+    rows = kvcache.quantize_kv_fp8((torch.randn(batch, length, 1, 512, generator=g) * 2).bfloat16(),
+                                   torch.randn(batch, length, 1, 64, generator=g).bfloat16(), pow2_scales=seed % 2 == 0)
+    q = torch.randn(batch, queries, heads, 512, generator=g).bfloat16()
+    qr = torch.randn(batch, queries, heads, 64, generator=g).bfloat16()
+    ids = torch.randint(0, length, (batch, queries, 1, topk), generator=g, dtype=torch.int32)
+    u = torch.rand(ids.shape, generator=g)
+    ids[u < 0.1] = -1
+    ids[u > 0.97] = length + 5
+    table = pool = None
+    if block:
+        per = length // block
+        blocks = batch * per + 3
+        table = torch.randperm(blocks, generator=g)[:batch * per].view(batch, per).int()
+        pool = torch.randint(0, 120, (blocks, block, 1, 656), generator=g, dtype=torch.uint8)
+        pool[table.reshape(-1).long()] = rows.reshape(batch * per, block, 1, 656)
+        table[:, 0] = torch.tensor([-1, blocks, 2 ** 31 - 1])[:batch]  # unbacked: slots of block 0 are masked
+        table[:, -1] = -7
+    ids[..., 0] = min(length - 1, max(block, 1) + 1)  # one backed slot in every row
+    return q, qr, ids, rows, table, pool
+
+
+@pytest.mark.parametrize("shape,block", [((1, 257, 128, 1024, 257), 0), ((2, 130, 16, 96, 64), 16),
+                                         ((3, 90, 48, 333, 40), 0), ((1, 300, 64, 192, 2048), 64),
+                                         ((3, 100, 32, 128, 300), 8)])
+def test_expanded_call_equals_bf16_call(shape, block):
+    from dsa_amd import api
+    from oracle import dsa_oracle as O
+
+    batch, queries, heads, length, topk = shape
+    assert api.expands_rows(shape)
+    q, qr, ids, rows, table, pool = _expanding_case(*shape, block, seed=heads)
+    kv, rope = O.dequant_fp8_rows(rows)
+    seen = ids.clone()
+    if block:  # the slots of unbacked blocks, masked by hand
+        entry = table.long()[torch.arange(batch)[:, None, None, None],
+                             (ids.long().clamp(0, length - 1) // block)]
+        seen[(entry < 0) | (entry >= pool.shape[0])] = -1
+    args = (q.cuda(), (rows if table is None else pool).cuda(), qr.cuda(), None, ids.cuda())
+    (got, launches) = dsa_amd.forward(*args, block_table=None if table is None else table.cuda(),
+                                      return_kernels=True)
+    assert launches[0].name == "expand_rows"
+    want = dsa_amd.forward(q.cuda(), kv.cuda(), qr.cuda(), rope.cuda(), seen.cuda())
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+def test_call_without_room_runs_on_the_rows(monkeypatch):
+    from dsa_amd import api
+
+    shape = (1, 257, 16, 512, 64)
+    q, qr, ids, rows, _, _ = _expanding_case(*shape, 0, seed=4)
+    args = (q.cuda(), rows.cuda(), qr.cuda(), None, ids.cuda())
+    want = dsa_amd.forward(*args, config=dsa_amd.plan_call(shape, None, 256, kv_fp8=True)[0])
+    monkeypatch.setattr(api, "_expanded_cache", lambda *_: None)
+    got, launches = dsa_amd.forward(*args, return_kernels=True)
+    assert all(l.name != "expand_rows" for l in launches)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
