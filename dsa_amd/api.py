@@ -209,7 +209,7 @@ def plan_call(shape, config=None, cores: int = 256, kv_fp8: bool = False, w_uv_d
     batch, queries, heads, _, _ = shape
     tokens = batch * queries
     if config.pv_cols == 128:
-        variant = "pp" if config.bm == 128 else "xs" if config.bn == 32 else "xp"
+        variant = "xp" if config.bn == 64 else "pp" if config.bm >= 64 else "xs"
     else:
         variant = "wide" if config.mfma == 32 else "narrow"
     threads, lds = (512, _PP_LDS_BYTES) if variant == "pp" else (256, _LDS_BYTES)

@@ -20,7 +20,10 @@ Ascend Cube/Vector pipeline; here the plan describes gfx950 workgroups:
                   Tuning.pv_cols): 512 (each wave: all columns for its own
                   rows) or 128 (the four waves split a 64-row tile's rows for
                   QK, exchange P through LDS and split the columns for PV;
-                  mfma 16, kv_waves 4, bm 16, 32 or 64).
+                  mfma 16, kv_waves 4, bm 16, 32 or 64).  With bn 32 and 4
+                  stages: the ping-pong kernel (bm 128, kv_waves 1, two groups of
+                  64 heads; bm 64, kv_waves 2, two streams of tiles) and the
+                  specialised waves (bm 16 or 32, kv_waves 2).
 
 Unlike the reference, shapes outside the table are accepted: the library's
 planner (``dsa_plan_for``) derives a plan for any supported shape.
@@ -135,24 +138,29 @@ _XP32 = dict(kv_waves=4, mfma=16, pv_cols=128)
 _PP = dict(kv_waves=1, stages=4, mfma=16, pv_cols=128)
 # Specialised waves (16 or 32 heads, 32-row tiles, four gather waves holding
 # three tiles in registers): ahead by 4-9 % on the 8- and 32-token decodes
-# (input sets cycled beyond the MALL) and the 16- and 128-query prefills
-# with 32 heads per group.
+# (input sets cycled beyond the MALL) and the prefills with 32 heads per group
+# (4096 queries of 32 heads: 894 against 951 us).
 _XS = dict(kv_waves=2, stages=4, mfma=16, pv_cols=128)
+# Ping-pong over tiles (64 heads, two tile streams; the same fields with bm 64):
+# the 64-head prefill 1,085 against 1,360 us per 4096 queries on wide<2,2>, the
+# 64-query prefill of 128 heads 57 against 62.5 us, the 32-token decode 41.0
+# against 43.5 us (split 4; the 8- and 16-token ones stay on the specialised
+# waves, 21.5 against 25.9 us at 8).
 SELECTED = {
     "decode_b1": Tuning(16, 64, 16, **_XP16),
     "decode_b8": Tuning(32, 32, 8, **_XS),
-    "decode_b32": Tuning(32, 32, 2, **_XS),
+    "decode_b32": Tuning(64, 32, 4, **_XS),
     "decode_tp8": Tuning(16, 64, 16, **_XP16),
     "prefill_q16": Tuning(32, 32, 4, **_XS),
-    "prefill_q64": Tuning(32, 64, 1, **_XP32),
+    "prefill_q64": Tuning(64, 32, 2, **_XS),
     "prefill_tp8": Tuning(16, 64, 2, fused_merge=True, **_XP16),
     "prefill_k512": Tuning(32, 32, 1, **_XS),
     "decode_b4_h128": Tuning(16, 64, 8, **_XP16),
     "prefill_b4_h128": Tuning(128, 32, 1, **_PP),
     "decode_b4_h64": Tuning(16, 64, 16, **_XP16),
-    "prefill_b4_h64": Tuning(64, 64, 1, kv_waves=2),
+    "prefill_b4_h64": Tuning(64, 32, 1, **_XS),
     "decode_b4_h32": Tuning(16, 64, 16, **_XP16),
-    "prefill_b4_h32": Tuning(32, 64, 1, **_XP32),
+    "prefill_b4_h32": Tuning(32, 32, 1, **_XS),
     "decode_b4_h16": Tuning(16, 64, 32, **_XP16),
     "prefill_b4_h16": Tuning(16, 64, 1, **_XP16),
     "c1_decode_b1": Tuning(16, 64, 16, **_XP16),

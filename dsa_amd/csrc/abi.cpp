@@ -77,7 +77,7 @@ int dsa_plan_check(const dsa_plan* plan, int B, int SQ, int H, int L, int TOPK) 
     const int ntiles = ceil_div(TOPK, bn);
     if (split < 1 || split > ntiles)
         return fail(-1, "split must be in [1, %d] for TOPK=%d (got %d)", ntiles, TOPK, split);
-    const int cap = dsa::fwd_index_cap(hpg, pv_cols);
+    const int cap = dsa::fwd_index_cap(hpg, bn, pv_cols);
     if (ceil_div(ntiles, split) * bn > cap)
         return fail(-1, "split %d leaves more than %d slots per workgroup (TOPK=%d)", split, cap, TOPK);
     if (plan->fused_merge != 0 && plan->fused_merge != 1)
@@ -122,39 +122,48 @@ int plan_impl(int B, int SQ, int H, int L, int TOPK, int num_cus, bool fp8, bool
     // measured 8 % under wide<4,1> per tile on the 4096- and 32768-token
     // prefills.  The specialised-wave variants (32-row tiles, gather waves)
     // measured within ±9 % of the column-split ones, ahead where a workgroup
-    // holds 32 heads.
+    // holds 32 heads.  The 64-head ping-pong variant (two tile streams) replaces
+    // wide<2,2> wherever 64-head workgroups pay (4096 queries of 64 heads 1,085
+    // against 1,360 us) and 128-head plans that fill less than half of the CUs
+    // (100 queries of 128 heads 72 against 83 us); it is behind at 8- and
+    // 16-token decodes (25.9 against 21.5 us at 8).  Its and the 128-head
+    // variants' costs were fitted by timing the old and the new choice on 187
+    // shapes whose plan they change (16 to 128 heads, 1 to 4096 tokens): median
+    // 10 % faster, one (20 tokens of 32 heads) 6 % slower.
     struct Variant {
         int hpg, kvw, bn, stages, mfma, pv_cols;
         bool bf16, fp8;
         double tile_cycles, epilogue_cycles;
+        double split_cycles = 0.0;  // further epilogue of a split: FP32 partial stores
     };
     static const Variant kVariants[] = {
-        {128, 1, 32, 4, 32, 512, true, false, 4400.0, 18000.0},  // wide<4,1,32,4>
-        {64, 2, 64, 2, 32, 512, true, false, 5000.0, 15000.0},   // wide<2,2,64,2>
+        {128, 1, 32, 4, 32, 512, true, false, 4400.0, 18000.0, 36000.0},  // wide<4,1,32,4>
+        {64, 2, 64, 2, 32, 512, true, false, 5000.0, 15000.0, 18000.0},   // wide<2,2,64,2>
         {64, 1, 64, 2, 16, 512, true, true, 7000.0, 6000.0},     // narrow<4,1>
         {32, 2, 64, 2, 16, 512, false, true, 4000.0, 10000.0},   // narrow<2,2>
         {16, 4, 64, 2, 16, 512, false, true, 2800.0, 10000.0},   // narrow<1,4>
         {32, 4, 64, 2, 16, 128, true, false, 3800.0, 6000.0},    // xp<2>: 32 heads, column-split PV
         {16, 4, 64, 2, 16, 128, true, false, 2700.0, 4000.0},    // xp<1>: 16 heads, column-split PV
-        {128, 1, 32, 4, 16, 128, true, false, 4000.0, 18000.0},  // ping-pong: 128 heads, eight waves
+        {128, 1, 32, 4, 16, 128, true, false, 3650.0, 18000.0, 36000.0},  // ping-pong: 128 heads, eight waves
+        {64, 2, 32, 4, 16, 128, true, false, 2350.0, 18000.0, 3000.0},  // ping-pong over tiles: 64 heads
         {32, 2, 32, 4, 16, 128, true, false, 1850.0, 6000.0},    // xs<2>: 32 heads, specialised waves
-        {16, 2, 32, 4, 16, 128, true, false, 1400.0, 4000.0},    // xs<1>: 16 heads, specialised waves
+        {16, 2, 32, 4, 16, 128, true, false, 1500.0, 4000.0},    // xs<1>: 16 heads, specialised waves
     };
     constexpr double kClockMHz = 2200.0, kPrologueCycles = 9000.0, kLaunchUs = 2.0;
     constexpr double kHbmBytesPerUs = 4.8e6, kCuBytesPerUs = 3.0e4;                // sustained gather rates
     constexpr double kMergeUs = 2.0, kMergeWgBytesPerUs = 4.2e4, kMergeBytesPerUs = 6.0e6;
     constexpr double kFp8TileCycles = 1200.0;  // expanding a 64-row fp8 tile to bf16 in LDS
-    constexpr double kFusedUs = 0.5, kFusedBytesPerUs = 3.0e4;  // in-kernel merge: count-in, one CU's read rate
+    constexpr double kFusedUs = 0.5, kFusedXsUs = 1.0, kFusedBytesPerUs = 3.0e4;  // in-kernel merge: count-in, one CU's read rate
     const int64_t tokens = (int64_t)B * SQ;
     const double gathered = (double)tokens * TOPK * (fp8 ? 656.0 : 1152.0);
-    double best = -1.0;
+    double best = -1.0, best_wg = 0.0;
     dsa_plan p{};
     for (const Variant& v : kVariants) {
         if (H % v.hpg) continue;
         if (fp8 ? !v.fp8 : !v.bf16) continue;
         const double tile_cycles = v.tile_cycles + (fp8 ? kFp8TileCycles : 0.0);
         const int ntiles = ceil_div(TOPK, v.bn);
-        const int min_split = ceil_div(ntiles * v.bn, dsa::fwd_index_cap(v.hpg, v.pv_cols));
+        const int min_split = ceil_div(ntiles * v.bn, dsa::fwd_index_cap(v.hpg, v.bn, v.pv_cols));
         const int64_t groups = tokens * (H / v.hpg);
         for (int split = min_split; split <= ntiles; ++split) {
             const int64_t wgs = groups * split;
@@ -164,7 +173,8 @@ int plan_impl(int B, int SQ, int H, int L, int TOPK, int num_cus, bool fp8, bool
                 break;  // larger splits need more partials still
             const double rounds = (double)((wgs + num_cus - 1) / num_cus);
             const double tiles = (double)ceil_div(ntiles, split);
-            const double wg_us = (kPrologueCycles + tiles * tile_cycles + v.epilogue_cycles) / kClockMHz;
+            const double wg_us = (kPrologueCycles + tiles * tile_cycles + v.epilogue_cycles +
+                                  (split > 1 ? v.split_cycles : 0.0)) / kClockMHz;
             const double active = (double)(wgs < num_cus ? wgs : num_cus);
             const double hbm = active * kCuBytesPerUs < kHbmBytesPerUs ? active * kCuBytesPerUs : kHbmBytesPerUs;
             double main_us = rounds * wg_us;
@@ -181,11 +191,19 @@ int plan_impl(int B, int SQ, int H, int L, int TOPK, int num_cus, bool fp8, bool
             int fused = 0;
             if (fuse && split > 1 && split <= kMaxFusedSplit && v.mfma == 16 && !(v.pv_cols == 128 && v.hpg != 16)) {
                 const double group_bytes = (double)split * v.hpg * 2056.0;
-                const double fused_cost = kLaunchUs + main_us + kFusedUs + group_bytes / kFusedBytesPerUs;
+                const double fused_cost =
+                    kLaunchUs + main_us + kFusedUs + (v.bn == 32 ? kFusedXsUs : 0.0) + group_bytes / kFusedBytesPerUs;
                 if (fused_cost < cost) cost = fused_cost, fused = 1;
             }
-            if (best < 0.0 || cost < best * 0.999) {
+            // Plans that the gather rate makes equal (prefill chunks, whose rows
+            // come from the caches rather than at that rate): the one with the
+            // cheaper workgroups.  32 heads, 4096 queries: specialised waves
+            // 894 us, column-split 951 us.
+            const bool equal = best >= 0.0 && split == p.split && cost < best * 1.001 &&
+                               rounds * wg_us < best_wg * 0.999;
+            if (best < 0.0 || cost < best * 0.999 || equal) {
                 best = cost;
+                best_wg = rounds * wg_us;
                 p.heads_per_group = v.hpg, p.kv_waves = v.kvw, p.tile_rows = v.bn, p.stages = v.stages;
                 p.mfma = v.mfma, p.split = split, p.fused_merge = fused, p.pv_cols = v.pv_cols;
             }

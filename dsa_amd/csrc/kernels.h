@@ -77,7 +77,7 @@ bool fwd_variant_exists(int heads_per_group, int kv_waves, int tile_rows, int st
 
 // Slots of the index cache of one workgroup of a variant (DSA_IDX_CAP, or
 // half of it where the LDS holds more per tile).
-int fwd_index_cap(int heads_per_group, int pv_cols);
+int fwd_index_cap(int heads_per_group, int tile_rows, int pv_cols);
 
 // Grid size (workgroups) of the main kernel for these params/plan.
 int64_t fwd_grid(const FwdParams& p);

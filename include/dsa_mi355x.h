@@ -84,7 +84,10 @@ extern "C" {
  *                     bf16 P tile through LDS and split the 512 output columns
  *                     for PV (mfma 16, kv_waves 4, tile_rows 64, stages 2,
  *                     heads_per_group 16, 32 or 64; with 64 heads a workgroup
- *                     holds at most 1024 slots).
+ *                     holds at most 1024 slots).  With tile_rows 32 and stages 4: the
+ *                     ping-pong kernel (heads_per_group 128 with kv_waves 1, or 64
+ *                     with kv_waves 2: two streams of tiles) and the specialised
+ *                     waves (heads_per_group 16 or 32, kv_waves 2).
  */
 typedef struct dsa_plan {
     int32_t heads_per_group;
