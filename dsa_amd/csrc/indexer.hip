@@ -20,14 +20,11 @@
 // waves sharing a query: 4 for single-query decode, 1 for prefill.
 //
 // Top-k kernel: one 1024-thread workgroup per query row.  A radix select over
-// order-preserving 32-bit keys of the logits finds the TOPK-th largest key T:
-// a 12-bit first digit over every candidate (4096 LDS bins, wide enough that
-// the atomics of clustered logits rarely collide), a 4-bit digit over the
-// LDS-cached upper halves of the keys, then two 8-bit digits over the few
-// entries that share T's upper 16 bits, gathered into LDS.  One sweep keeps
-// every s with key > T and the lowest-s ties == T, written in ascending
-// order.  A row of up to 65536 candidates is read from memory once, plus its
-// gathered entries.
+// order-preserving 32-bit keys of the logits finds the TOPK-th largest key T
+// and one sweep keeps every s with key > T and the lowest-s ties == T, written
+// in ascending order.  Rows of up to 65536 candidates are read from memory
+// once, into registers (topk_registers); longer ones are read once per digit
+// (topk_select).
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include <float.h>
@@ -229,25 +226,32 @@ __global__ __launch_bounds__(256, 1) void indexer_logits_kernel(IndexerParams p)
 // ------------------------------------------------------------------ top-k
 constexpr int kTopkThreads = 1024;
 constexpr int kTopkWaves = kTopkThreads / 64;
-constexpr int kChunk = 256;        // entries one wave covers per step: 4 consecutive per lane
-constexpr int kCacheKeys = 65536;  // bits 31..16 of every candidate's key cached in LDS (128 KiB)
-constexpr int kBins0 = 4096;       // first digit: key bits 31..20 (sign, exponent, 3 mantissa bits)
-constexpr int kCandCap = 1536;     // entries sharing T's upper 16 bits kept in LDS as (s, key)
+constexpr int kChunk = 256;       // entries one wave covers per step: 4 consecutive per lane
+constexpr int kRegKeys = 65536;   // longest row held in registers (64 keys per thread)
+constexpr int kBins0 = 4096;      // first digit: key bits 31..20 (sign, exponent, 3 mantissa bits)
+constexpr int kCandCap = 1536;    // entries sharing T's upper 16 bits kept in LDS as (s, key)
+constexpr int kStageOut = 4096;   // largest TOPK whose row is assembled in LDS
 
 struct TopkShared {
-    __attribute__((aligned(16))) uint16_t hi16[kCacheKeys];
-    uint32_t hist[kBins0];  // digit histograms; afterwards 2 flag bits per cached s
-    uint32_t cand_s[kCandCap];
-    uint32_t cand_key[kCandCap];
+    uint32_t hist[kBins0];  // digit histograms; rows in registers: afterwards the selected s
+    union {
+        struct {  // topk_select
+            uint32_t cand_s[kCandCap];
+            uint32_t cand_key[kCandCap];
+        };
+        uint32_t hist_low[2][1024];  // topk_registers: key bits 19..10, 9..0
+    };
     uint32_t wgt[kTopkWaves];  // per wave segment: entries with key > T
     uint32_t weq[kTopkWaves];  // per wave segment: entries with key == T
     uint32_t word[4];
 };
 
-// Order-preserving map of a float to an unsigned key (larger float, larger key).
+// Order-preserving map of a float to an unsigned key (larger float, larger
+// key): all bits of a negative flipped, the sign of any other set (one shift and
+// one three-input bitwise instruction).
 __device__ __forceinline__ uint32_t float_key(float f) {
     const uint32_t u = __float_as_uint(f);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+    return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
 }
 
 __device__ __forceinline__ uint64_t lanes_below(int lane) { return lane == 0 ? 0ull : (~0ull >> (64 - lane)); }
@@ -258,14 +262,22 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
     return v;
 }
 
-// Inclusive prefix sum across the wave (lane order).
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, int lane) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(v, d);
-        if (lane >= d) v += o;
-    }
-    return v;
+// Inclusive prefix sum across the wave (lane order): DPP row shifts within the
+// 16-lane rows, then the row totals broadcast to the rows behind.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ uint32_t row_incl_scan(uint32_t v) {
+    v += dpp_or_zero<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+    v += dpp_or_zero<0x112, 0xf>(v);
+    v += dpp_or_zero<0x114, 0xf>(v);
+    return v + dpp_or_zero<0x118, 0xf>(v);
+}
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+    v = row_incl_scan(v);
+    v += dpp_or_zero<0x142, 0xa>(v);         // row_bcast:15 into rows 1 and 3
+    return v + dpp_or_zero<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
 }
 
 // One row of logits behind a range-checked buffer descriptor: reads at or past
@@ -310,39 +322,26 @@ __device__ __forceinline__ uint32_t valid4(int s, int hi) {
     return left >= 4 ? 15u : (left <= 0 ? 0u : (1u << left) - 1u);
 }
 
-// Upper key halves of entries s .. s + 3 of one wave step (s = base + 4 lane,
-// base a multiple of kChunk below hi): from the LDS cache, or from memory.
-template <bool CACHED>
-__device__ __forceinline__ void upper4(const TopkShared& sh, const Row& row, int base, int s, uint32_t h[4]) {
-    if constexpr (CACHED) {
-        (void)base;
-        const uint2 v = *reinterpret_cast<const uint2*>(&sh.hi16[s]);
-        h[0] = v.x & 0xffffu;
-        h[1] = v.x >> 16;
-        h[2] = v.y & 0xffffu;
-        h[3] = v.y >> 16;
-    } else {
+// Upper key halves of entries s .. s + 3.
+__device__ __forceinline__ void upper4(const Row& row, int s, uint32_t h[4]) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) h[j] = row.key(s + j) >> 16;
-    }
+    for (int j = 0; j < 4; ++j) h[j] = row.key(s + j) >> 16;
 }
 
 // Per row: the threshold key T (the K-th largest key) and the number of
 // entries equal to T to take, found digit by digit, then one sweep that
 // writes the selected s in ascending order.  Each wave owns a contiguous
 // segment of s, walked kChunk entries at a time.
-//   digit 0, bits 31..20: one read of the row; caches the keys' bits 31..16
-//   digit 1, bits 19..16: entries of digit 0's bin, from the cache; also
-//           counts per segment the entries whose upper 16 bits exceed T's
+//   digit 0, bits 31..20: one read of the row
+//   digit 1, bits 19..16: entries of digit 0's bin; also counts per segment
+//           the entries whose upper 16 bits exceed T's
 //   gather: the entries sharing T's upper 16 bits (typically a few hundred)
 //           as (s, key) into LDS -- one batch of independent loads
 //   digits 2, 3, bits 15..8 and 7..0: over the gathered entries, which then
 //           get flags (key > T, key == T) and per-segment counts
 //   sweep: the segment counts place every wave's writes.
-// CACHED = false (rows longer than the cache) reads the row from memory in
-// every pass; a 16-bit prefix shared by more than kCandCap entries is
-// resolved over the whole row, reading keys from memory.
-template <bool CACHED>
+// Every pass reads the row from memory (rows longer than kRegKeys); a 16-bit
+// prefix shared by more than kCandCap entries is resolved over the whole row.
 __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int32_t* __restrict__ dst, int n,
                                             int K) {
     const int tid = threadIdx.x;
@@ -352,7 +351,7 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
     const int lo = min(wave * seg, n), hi = min(lo + seg, n);  // this wave's entries [lo, hi)
     constexpr int U = 4;  // wave steps per loop iteration (loads in flight)
 
-    // ---- digit 0 (bits 31..20) over every candidate; caches bits 31..16
+    // ---- digit 0 (bits 31..20) over every candidate
     for (int i = tid; i < kBins0; i += kTopkThreads) sh.hist[i] = 0;
     if (tid < kTopkWaves) sh.weq[tid] = 0;
     if (tid == 0) sh.word[2] = 0;
@@ -365,8 +364,6 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
 #pragma unroll
         for (int c = 0; c < 2 * U * 4; ++c) {
             const int s = base + c * 64 + lane;
-            if constexpr (CACHED)
-                if (base + (c / 4) * kChunk < hi) sh.hi16[s] = (uint16_t)(k[c] >> 16);  // step inside the cache
             if (s < hi) atomicAdd(&sh.hist[k[c] >> 20], 1u);
         }
     }
@@ -380,7 +377,7 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
             c[j] = sh.hist[kBins0 - 1 - 4 * tid - j];
             mine += c[j];
         }
-        const uint32_t incl = wave_incl_scan(mine, lane);
+        const uint32_t incl = wave_incl_scan(mine);
         if (lane == 63) sh.wgt[wave] = incl;
         __syncthreads();
         uint32_t above = incl - mine;
@@ -409,7 +406,7 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if (base + u * kChunk < hi) {
-                    upper4<CACHED>(sh, row, base + u * kChunk, base + u * kChunk + 4 * lane, h[u]);
+                    upper4(row, base + u * kChunk + 4 * lane, h[u]);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) h[u][j] = 0;
@@ -438,7 +435,7 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
         uint32_t c = 0;
         if (lane < 16)
             for (int w = 0; w < kTopkWaves; ++w) c += sh.hist[w * 16 + 15 - lane];
-        const uint32_t above = wave_incl_scan(c, lane) - c;
+        const uint32_t above = wave_incl_scan(c) - c;
         if (lane < 16 && above < need && above + c >= need) {
             sh.word[0] = 15 - lane;
             sh.word[1] = above;
@@ -465,7 +462,7 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if (base + u * kChunk < hi) {
-                    upper4<CACHED>(sh, row, base + u * kChunk, base + u * kChunk + 4 * lane, h[u]);
+                    upper4(row, base + u * kChunk + 4 * lane, h[u]);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) h[u][j] = 0;
@@ -517,7 +514,7 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
                 c[j] = sh.hist[255 - (4 * lane + j)];
                 sum += c[j];
             }
-            uint32_t above = wave_incl_scan(sum, lane) - sum;
+            uint32_t above = wave_incl_scan(sum) - sum;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 if (above < need && above + c[j] >= need) {
@@ -535,9 +532,7 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
     }
     const uint32_t thr = prefix;
 
-    // ---- segment counts (and, for a cached row, flags) of the entries sharing pre16
-    if (CACHED && gathered)
-        for (int i = tid; i < kBins0; i += kTopkThreads) sh.hist[i] = 0;
+    // ---- segment counts of the entries sharing pre16
     __syncthreads();
     if (gathered) {
         for (int i = tid; i < (int)in16; i += kTopkThreads) {
@@ -545,10 +540,6 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
             const int w = (int)s / seg;
             if (u > thr) atomicAdd(&sh.wgt[w], 1u);
             if (u == thr) atomicAdd(&sh.weq[w], 1u);
-            if constexpr (CACHED) {
-                const uint32_t f = (u > thr ? 1u : 0u) | (u == thr ? 2u : 0u);
-                if (f) atomicOr(&sh.hist[s >> 4], f << (2 * (s & 15)));
-            }
         }
     } else {
         uint32_t ng = 0, ne = 0;
@@ -573,17 +564,12 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
         ties += sh.weq[w];
     }
     pos += min(ties, need);
-    const bool flags = CACHED && gathered;
     for (int base = lo; base < hi; base += U * kChunk) {
-        uint32_t h[U][4], f8[U];
+        uint32_t h[U][4];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            f8[u] = 0;
             if (base + u * kChunk < hi) {
-                const int s = base + u * kChunk + 4 * lane;
-                upper4<CACHED>(sh, row, base + u * kChunk, s, h[u]);
-                // flag bits of entries s .. s + 3: byte (s % 16) / 4 of flag word s / 16
-                if (flags) f8[u] = (sh.hist[s >> 4] >> (8 * (lane & 3))) & 0xffu;
+                upper4(row, base + u * kChunk + 4 * lane, h[u]);
             } else {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) h[u][j] = 0;
@@ -594,13 +580,8 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
             const int s = base + u * kChunk + 4 * lane;
             const uint32_t vm = valid4(s, hi);
             const uint32_t mid = mask_eq4(h[u], pre16) & vm;  // share T's upper 16 bits
-            const uint32_t f = f8[u];
-            // de-interleave the flags: bit 2j = key > T, bit 2j + 1 = key == T
-            const uint32_t fgt = (f & 1u) | ((f >> 1) & 2u) | ((f >> 2) & 4u) | ((f >> 3) & 8u);
-            const uint32_t feq = ((f >> 1) & 1u) | ((f >> 2) & 2u) | ((f >> 3) & 4u) | ((f >> 4) & 8u);
-            uint32_t gtm = (mask_gt4(h[u], pre16) & vm) | (mid & fgt);
-            uint32_t eqm = mid & feq;
-            if (!flags && __ballot(mid != 0u)) {  // keys of the entries sharing pre16, from memory
+            uint32_t gtm = mask_gt4(h[u], pre16) & vm, eqm = 0;
+            if (__ballot(mid != 0u)) {  // keys of the entries sharing pre16, from memory
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const uint32_t key = row.key(s + j);
@@ -638,10 +619,186 @@ __device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int3
     }
 }
 
-__global__ __launch_bounds__(kTopkThreads, 1) void indexer_topk_kernel(const float* __restrict__ logits,
-                                                                      const int32_t* __restrict__ len,
-                                                                      int32_t* __restrict__ out, int L, int K) {
-    __shared__ TopkShared sh;
+// The bin holding the need-th largest of the entries counted in hist[1024],
+// found by every wave for itself (16 bins per lane, no barrier): need becomes
+// the entries to take from that bin, count the entries in it.
+__device__ __forceinline__ uint32_t find_bin1024(const uint32_t* hist, int lane, uint32_t& need, uint32_t& count) {
+    uint32_t c[16], mine = 0;  // bins 1008 - 16 lane .. 1023 - 16 lane: lane 0 holds the top ones
+    const uint4* src = reinterpret_cast<const uint4*>(hist + 1008 - 16 * lane);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint4 v = src[q];
+        c[4 * q] = v.x, c[4 * q + 1] = v.y, c[4 * q + 2] = v.z, c[4 * q + 3] = v.w;
+        mine += v.x + v.y + v.z + v.w;
+    }
+    const uint32_t incl = wave_incl_scan(mine);
+    uint32_t above = incl - mine, bin = 0, found = 0, left = 0;
+#pragma unroll
+    for (int j = 15; j >= 0; --j) {
+        const bool here = above < need && above + c[j] >= need;  // in one lane, for one j
+        bin = here ? (uint32_t)(1008 - 16 * lane + j) : bin;
+        left = here ? need - above : left;
+        found = here ? c[j] : found;
+        above += c[j];
+    }
+    const int src_lane = __builtin_ctzll(__ballot(found != 0u));
+    need = (uint32_t)__builtin_amdgcn_readlane((int)left, src_lane);
+    count = (uint32_t)__builtin_amdgcn_readlane((int)found, src_lane);
+    return (uint32_t)__builtin_amdgcn_readlane((int)bin, src_lane);
+}
+
+// Sum of v[0 .. wave) over the kTopkWaves entries of an LDS array, per wave.
+__device__ __forceinline__ uint32_t waves_below(const uint32_t* v, int wave, int lane) {
+    const uint32_t incl = row_incl_scan(v[lane & (kTopkWaves - 1)]);
+    return wave == 0 ? 0u : (uint32_t)__builtin_amdgcn_readlane((int)incl, wave - 1);
+}
+
+// The selection of a row of n <= 64 * 16 * KPT candidates held in registers:
+// wave w owns s in [w * 64 * steps, (w + 1) * 64 * steps), lane l entries
+// l, l + 64, ... of it, so every load is 256 contiguous bytes and ascending s
+// is step, then lane.  The row is read once, all loads in flight; three digits
+// (12, 10, 10 bits) of LDS histogram fix T, ballots count and place the output.
+// Bound by instruction issue (about 35 per 64 entries over the five passes);
+// with 32 keys per thread or fewer two workgroups share a CU, one reading or in
+// a barrier while the other counts.  Measured: see launch_indexer_topk.
+// Slots past n hold key 0 and the largest s: n > K, so they are never taken.
+template <int KPT>
+__device__ __forceinline__ void topk_registers(TopkShared& sh, const Row& row, int32_t* __restrict__ dst, int n,
+                                               int K) {
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int G = 4;  // steps per uniform skip
+    // 64-entry steps of a wave, a multiple of G, <= KPT
+    const int steps = (n + G * kTopkThreads - 1) / (G * kTopkThreads) * G;
+    const int lo = wave * 64 * steps;
+    const int mine = lo < n ? steps : 0;  // steps this wave runs
+
+    uint32_t key[KPT];
+    // Between the phases: values derived from the keys are recomputed, not kept
+    // in registers beside them.
+    auto opaque = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < KPT; ++c) asm volatile("" : "+v"(key[c]));
+    };
+#define TOPK_STEPS(c)                                         \
+    _Pragma("unroll") for (int c0 = 0; c0 < KPT; c0 += G)     \
+        if (c0 < mine) _Pragma("unroll") for (int c = c0; c < c0 + G; ++c)
+#pragma unroll
+    for (int c = 0; c < KPT; ++c) key[c] = 0;
+    const int voff = (lo + lane) * 4;
+    TOPK_STEPS(c) key[c] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(row.rs, voff + c * 256, 0, 0);
+    reinterpret_cast<uint4*>(sh.hist)[tid] = uint4{0, 0, 0, 0};
+    static_assert(kBins0 == 4 * kTopkThreads, "four first-digit bins per thread");
+    if (tid < 512) reinterpret_cast<uint4*>(sh.hist_low)[tid] = uint4{0, 0, 0, 0};
+    __syncthreads();
+
+    // ---- digit 0 (bits 31..20)
+    opaque();
+    if (lo + 64 * steps <= n) {  // every slot holds an entry
+        TOPK_STEPS(c) {
+            key[c] = float_key(__uint_as_float(key[c]));
+            atomicAdd(&sh.hist[key[c] >> 20], 1u);
+        }
+    } else {
+        TOPK_STEPS(c) {
+            const bool in = lo + c * 64 + lane < n;
+            key[c] = in ? float_key(__uint_as_float(key[c])) : 0u;
+            if (in) atomicAdd(&sh.hist[key[c] >> 20], 1u);
+        }
+    }
+    __syncthreads();
+    uint32_t need = (uint32_t)K;  // entries still to take among those matching the digits so far
+    {
+        // thread tid owns bins kBins0 - 4 - 4 tid .. + 3, counted from the top
+        const uint4 v = *reinterpret_cast<const uint4*>(&sh.hist[kBins0 - 4 - 4 * tid]);
+        const uint32_t c[4] = {v.w, v.z, v.y, v.x};
+        const uint32_t sum = v.x + v.y + v.z + v.w;
+        const uint32_t incl = wave_incl_scan(sum);
+        if (lane == 63) sh.wgt[wave] = incl;
+        __syncthreads();
+        uint32_t above = incl - sum + waves_below(sh.wgt, wave, lane);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (above < need && above + c[j] >= need) {  // exactly one (thread, j) crosses
+                sh.word[0] = (uint32_t)(kBins0 - 1 - 4 * tid - j);
+                sh.word[1] = above;
+            }
+            above += c[j];
+        }
+        __syncthreads();
+    }
+    const uint32_t bin0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.word[0]);
+    need -= (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.word[1]);
+
+    // ---- digits 1, 2 (bits 19..10, 9..0)
+    uint32_t count;
+    opaque();
+    TOPK_STEPS(c) if (key[c] >> 20 == bin0) atomicAdd(&sh.hist_low[0][(key[c] >> 10) & 1023u], 1u);
+    __syncthreads();
+    const uint32_t pre22 = bin0 << 10 | find_bin1024(sh.hist_low[0], lane, need, count);
+    opaque();
+    TOPK_STEPS(c) if (key[c] >> 10 == pre22) atomicAdd(&sh.hist_low[1][key[c] & 1023u], 1u);
+    __syncthreads();
+    const uint32_t thr = pre22 << 10 | find_bin1024(sh.hist_low[1], lane, need, count);
+    const bool all_ties = count == need;  // every entry equal to T is taken (uniform)
+    opaque();
+
+    // ---- entries per wave: >= T with all_ties, else > T and == T
+    uint32_t ngt = 0, neq = 0;
+    if (all_ties) {
+        TOPK_STEPS(c) ngt += (uint32_t)__popcll(__ballot(key[c] >= thr));
+    } else {
+        TOPK_STEPS(c) {
+            ngt += (uint32_t)__popcll(__ballot(key[c] > thr));
+            neq += (uint32_t)__popcll(__ballot(key[c] == thr));
+        }
+    }
+    if (lane == 0) {
+        sh.wgt[wave] = ngt;
+        sh.weq[wave] = neq;
+    }
+    __syncthreads();
+    uint32_t pos = waves_below(sh.wgt, wave, lane);
+    opaque();
+
+    // ---- output, ascending s (assembled in LDS where it fits)
+    const bool staged = K <= kStageOut;
+    auto put = [&](bool take, int c) __attribute__((always_inline)) {
+        const uint64_t m = __ballot(take);
+        if (take) {
+            const uint32_t at =
+                __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, pos));
+            if (staged) sh.hist[at] = (uint32_t)(lo + c * 64 + lane);
+            else dst[at] = lo + c * 64 + lane;
+        }
+        pos += (uint32_t)__popcll(m);
+    };
+    if (all_ties) {
+        TOPK_STEPS(c) put(key[c] >= thr, c);
+    } else {
+        uint32_t ties = waves_below(sh.weq, wave, lane);
+        pos += min(ties, need);
+        TOPK_STEPS(c) {
+            const bool tie = key[c] == thr;
+            const uint64_t m = __ballot(tie);
+            put(tie ? ties + lane_rank(m) < need : key[c] > thr, c);
+            ties += (uint32_t)__popcll(m);
+        }
+    }
+#undef TOPK_STEPS
+    if (staged) {
+        __syncthreads();
+        for (int j = tid; j < K; j += kTopkThreads) dst[j] = (int32_t)sh.hist[j];
+    }
+}
+
+// KPT: keys per thread of rows held in registers; LONG: rows may exceed
+// kRegKeys (L does).
+template <int KPT, bool LONG>
+__global__ __launch_bounds__(kTopkThreads, KPT <= 32 ? 8 : 4) void indexer_topk_kernel(
+    const float* __restrict__ logits, const int32_t* __restrict__ len, int32_t* __restrict__ out, int L, int K) {
+    __shared__ __attribute__((aligned(16))) TopkShared sh;
     const int r = blockIdx.x;
     const int n = min(max(len[r], 0), L);
     int32_t* dst = out + (int64_t)r * K;
@@ -651,15 +808,19 @@ __global__ __launch_bounds__(kTopkThreads, 1) void indexer_topk_kernel(const flo
     }
     const Row row{__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(logits + (int64_t)r * L), (short)0, n * 4,
                                                     0x00020000)};
-    if (n <= kCacheKeys)
-        topk_select<true>(sh, row, dst, n, K);
-    else
-        topk_select<false>(sh, row, dst, n, K);
+    if constexpr (LONG) {
+        if (n > kRegKeys) {
+            topk_select(sh, row, dst, n, K);
+            return;
+        }
+    }
+    topk_registers<KPT>(sh, row, dst, n, K);
 }
 
 // ------------------------------------------------ segmented top-k (few rows)
-// With few rows, one 1024-thread workgroup per row leaves most CUs idle and is
-// bound by its own VALU issue.  The segmented path splits every row over
+// With few long rows, one 1024-thread workgroup per row leaves most CUs idle and
+// is bound by its own VALU issue (rows of up to kSegMinKeys entries are faster
+// in one workgroup's registers).  The segmented path splits every row over
 // kSegWgs workgroups of 256 threads, each owning the contiguous segment
 // [p * seg, (p + 1) * seg) of s, in three launches (the kernel boundaries are
 // the only synchronisation; the workspace needs no initialisation):
@@ -677,6 +838,7 @@ __global__ __launch_bounds__(kTopkThreads, 1) void indexer_topk_kernel(const flo
 constexpr int kSegWgs = 8;          // workgroups per row
 constexpr int kSegThreads = 256;
 constexpr int kSegMaxRows = 32;     // rows * kSegWgs workgroups at most: 256
+constexpr int kSegMinKeys = kIndexerSegMinKeys;
 constexpr int kSegCandCap = 8192;   // candidates resolved from LDS; more are read from the workspace
 constexpr int kSegKeys = 16;        // keys per thread in flight (4096 per workgroup and batch)
 
@@ -773,7 +935,7 @@ __global__ __launch_bounds__(kSegThreads) void seg_cand_kernel(const float* __re
         for (int q = 0; q < kSegWgs; ++q) v[q] = w.coarse(q)[kCoarse - 1 - lane];
 #pragma unroll
         for (int q = 0; q < kSegWgs; ++q) sum += v[q];
-        uint32_t above = wave_incl_scan(sum, lane) - sum;
+        uint32_t above = wave_incl_scan(sum) - sum;
         const bool cross = above < (uint32_t)K && above + sum >= (uint32_t)K;  // one lane
         const uint64_t m = __ballot(cross);
         const int src = __builtin_ctzll(m);
@@ -784,7 +946,7 @@ __global__ __launch_bounds__(kSegThreads) void seg_cand_kernel(const float* __re
         sum = 0;
 #pragma unroll
         for (int q = 0; q < kSegWgs; ++q) sum += v[q];
-        uint32_t above2 = above + wave_incl_scan(sum, lane) - sum;
+        uint32_t above2 = above + wave_incl_scan(sum) - sum;
         if (above2 < (uint32_t)K && above2 + sum >= (uint32_t)K) {
             word[0] = cbin * (kBins0 / kCoarse) + (kBins0 / kCoarse - 1 - lane);
             word[1] = above2;
@@ -829,7 +991,7 @@ __global__ __launch_bounds__(kSegThreads) void seg_cand_kernel(const float* __re
 // per-thread count.  Uses tot[kSegThreads / 64] of LDS.
 __device__ __forceinline__ void block_prefix(uint32_t c, uint32_t* tot, uint32_t& before, uint32_t& total) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t incl = wave_incl_scan(c, lane);
+    const uint32_t incl = wave_incl_scan(c);
     if (lane == 63) tot[wave] = incl;
     __syncthreads();
     before = incl - c;
@@ -968,7 +1130,7 @@ __global__ __launch_bounds__(kSegThreads) void seg_emit_kernel(const float* __re
             cc[j] = hist[255 - (4 * lane + j)];
             sum += cc[j];
         }
-        uint32_t a = wave_incl_scan(sum, lane) - sum;
+        uint32_t a = wave_incl_scan(sum) - sum;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             if (a < need && a + cc[j] >= need) word[2] = (uint32_t)(255 - (4 * lane + j));
@@ -1084,6 +1246,26 @@ int launch_indexer_logits(const IndexerParams& p, hipStream_t stream) {
     return (int)hipErrorInvalidValue;
 }
 
+// The least register kernel that holds a row of L (fewer keys per thread leave
+// less to unroll and skip).  Against the same selection reading LDS-cached key
+// halves, one workgroup per CU: 4096 causal rows of 32768 202 us instead of 345,
+// 128 rows of 65536 23 us instead of 36, 512 rows of 16384 16 us instead of 32.
+int launch_indexer_topk(const float* logits, const int32_t* len, int32_t* indices, int rows, int L, int topk,
+                        hipStream_t stream) {
+    const dim3 grid((unsigned)rows), block(kTopkThreads);
+    if (L <= 8 * kTopkThreads)
+        hipLaunchKernelGGL((indexer_topk_kernel<8, false>), grid, block, 0, stream, logits, len, indices, L, topk);
+    else if (L <= 16 * kTopkThreads)
+        hipLaunchKernelGGL((indexer_topk_kernel<16, false>), grid, block, 0, stream, logits, len, indices, L, topk);
+    else if (L <= 32 * kTopkThreads)
+        hipLaunchKernelGGL((indexer_topk_kernel<32, false>), grid, block, 0, stream, logits, len, indices, L, topk);
+    else if (L <= kRegKeys)
+        hipLaunchKernelGGL((indexer_topk_kernel<64, false>), grid, block, 0, stream, logits, len, indices, L, topk);
+    else
+        hipLaunchKernelGGL((indexer_topk_kernel<64, true>), grid, block, 0, stream, logits, len, indices, L, topk);
+    return (int)hipGetLastError();
+}
+
 int64_t indexer_topk_ws_bytes(int rows, int L) {
     if (rows > kSegMaxRows) return 0;
     return (int64_t)rows * seg_row_words(L) * 4;
@@ -1091,19 +1273,14 @@ int64_t indexer_topk_ws_bytes(int rows, int L) {
 
 int launch_indexer_topk_seg(const float* logits, const int32_t* len, int32_t* indices, void* ws, int rows, int L,
                             int topk, hipStream_t stream) {
+    // 8 rows of 32768: 14.6 us in one workgroup each, 18.5 us segmented; of 65536: 21.6 and 19.7 us
+    if (L <= kSegMinKeys) return launch_indexer_topk(logits, len, indices, rows, L, topk, stream);
     uint32_t* w = static_cast<uint32_t*>(ws);
     const dim3 grid((unsigned)rows, (unsigned)kSegWgs);
     hipLaunchKernelGGL(seg_hist_kernel, grid, dim3(kSegThreads), 0, stream, logits, len, indices, w, L, topk);
     hipLaunchKernelGGL(seg_cand_kernel, grid, dim3(kSegThreads), 0, stream, logits, len, w, L, topk);
     hipLaunchKernelGGL(seg_emit_kernel, grid, dim3(kSegThreads), 0, stream, logits, len, indices,
                        static_cast<const uint32_t*>(w), L, topk);
-    return (int)hipGetLastError();
-}
-
-int launch_indexer_topk(const float* logits, const int32_t* len, int32_t* indices, int rows, int L, int topk,
-                        hipStream_t stream) {
-    hipLaunchKernelGGL(indexer_topk_kernel, dim3((unsigned)rows), dim3(kTopkThreads), 0, stream, logits, len,
-                       indices, L, topk);
     return (int)hipGetLastError();
 }
 

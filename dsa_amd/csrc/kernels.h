@@ -149,6 +149,10 @@ int launch_indexer_logits(const IndexerParams& p, hipStream_t stream);
 int launch_indexer_topk(const float* logits, const int32_t* len, int32_t* indices, int rows, int L, int topk,
                         hipStream_t stream);
 
+// Rows up to this length are selected by one workgroup also where a workspace
+// for the segmented selection is given.
+constexpr int kIndexerSegMinKeys = 32768;
+
 // Workspace bytes of the segmented selection (several workgroups per row, for
 // few rows); 0 when rows are too many for it to pay.
 int64_t indexer_topk_ws_bytes(int rows, int L);

@@ -18,6 +18,7 @@ from . import _lib
 
 INDEX_DIM = 128
 INDEX_HEADS = (32, 64)
+SEGMENTED_MIN_LENGTH = 32768  # rows up to this length take one workgroup (kIndexerSegMinKeys)
 
 
 def _device_ok(device, tensors):
@@ -63,8 +64,9 @@ def indexer_topk(logits, lengths, topk: int, *, segmented: bool = True):
     """``indices [B, SQ, 1, topk]`` int32: per row the ``topk`` largest logits among
     ``s < lengths`` (ties: lower ``s`` first), ascending, padded with -1.
 
-    With few rows (``B * SQ <= 32``) and ``segmented`` the selection splits every
-    row over 8 workgroups (three launches, same result bit for bit)."""
+    With few long rows (``B * SQ <= 32``, ``L > 32768``) and ``segmented`` the
+    selection splits every row over 8 workgroups (three launches, same result
+    bit for bit); shorter rows are selected in one workgroup's registers."""
     if type(topk) is not int or topk <= 0:
         raise ValueError("topk must be a positive int")
     if logits.dim() != 3 or min(logits.shape) <= 0:
@@ -80,8 +82,9 @@ def indexer_topk(logits, lengths, topk: int, *, segmented: bool = True):
     stream = torch.cuda.current_stream(device).cuda_stream
     p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
     lib = _lib.load()
-    # few rows: the segmented selection (8 workgroups per row) over a scratch workspace
-    ws_bytes = lib.dsa_indexer_topk_ws_bytes(batch, queries, length, topk) if segmented else 0
+    # few long rows: the segmented selection (8 workgroups per row) over a scratch workspace
+    split_rows = segmented and length > SEGMENTED_MIN_LENGTH
+    ws_bytes = lib.dsa_indexer_topk_ws_bytes(batch, queries, length, topk) if split_rows else 0
     with torch.cuda.device(device):
         if ws_bytes > 0:
             ws = torch.empty(ws_bytes, device=device, dtype=torch.uint8)

@@ -358,8 +358,8 @@ int dsa_indexer_topk(const float* logits, const int32_t* lengths, int32_t* indic
 
 /*
  * dsa_indexer_topk with a workspace (no reference counterpart, like the
- * indexer).  With few rows (B * SQ <= 32) one workgroup per row leaves most
- * CUs idle; given `workspace` of at least dsa_indexer_topk_ws_bytes bytes
+ * indexer).  With few long rows (B * SQ <= 32, L > 32768) one workgroup per row
+ * leaves most CUs idle; given `workspace` of at least dsa_indexer_topk_ws_bytes bytes
  * (16-byte aligned, any contents), every row is split over 8 workgroups in
  * three launches instead.  Same result bit for bit.  A NULL workspace, or a
  * size query that returns 0 (many rows), selects dsa_indexer_topk's kernel.
