@@ -579,14 +579,34 @@ int dsa_indexer_logits(const uint16_t* q_idx, const uint16_t* k_idx, const float
     p.ks = (int64_t)SQ * HI <= 64 ? 4 : ((int64_t)SQ * HI <= 128 ? 2 : 1);
     p.tgroups = ceil_div(SQ, 256 / HI / p.ks);
     p.ntiles = ceil_div(L, 64 * p.ks);
-    // About 1024 / ks workgroups (a stage of ks x 16 KiB, two stages per
-    // workgroup): decode spreads one query's keys over many CUs, prefill keeps
-    // every key stage of a query group in one workgroup.
-    const int64_t work = (int64_t)B * p.tgroups * p.ntiles;
-    const int64_t target = 1024 / p.ks;
-    p.tiles_per_wg = (int)((work + target - 1) / target);
-    if (p.tiles_per_wg < 1) p.tiles_per_wg = 1;
-    if (p.tiles_per_wg > p.ntiles) p.tiles_per_wg = p.ntiles;
+    // Stages per workgroup.  With at least 32 each in 2048 / ks workgroups, that
+    // many: the end of the launch is even (64 x 2 queries over 65536 keys 208 us
+    // against 216 us in half as many).  Below that a range's start counts: the
+    // split whose rounds of resident workgroups (two per CU, one where its two
+    // stages of ks x 16 KiB fill the LDS) take the least time, the start taken
+    // as kStartStages stages (3 x 700 queries over 5000 keys 150 us against
+    // 162 us in 1024 workgroups, 300 over 2000 16.8 against 19.2 us).
+    const int64_t groups = (int64_t)B * p.tgroups, work = groups * p.ntiles;
+    if (work * p.ks >= 2048 * 32) {
+        p.tiles_per_wg = (int)((work * p.ks + 2047) / 2048);
+        if (p.tiles_per_wg > p.ntiles) p.tiles_per_wg = p.ntiles;
+    } else {
+        constexpr int kCus = 256, kStartStages = 3;
+        const int64_t slots = kCus * (p.ks == 4 ? 1 : 2);
+        int64_t best = -1;
+        for (int64_t rounds = 1; rounds <= 8; ++rounds) {  // the most ranges that fit in so many rounds
+            int64_t ranges = rounds * slots / groups;
+            if (ranges < 1) ranges = 1;
+            if (ranges > p.ntiles) ranges = p.ntiles;
+            const int tiles = (int)((p.ntiles + ranges - 1) / ranges);
+            const int64_t wgs = groups * ((p.ntiles + tiles - 1) / tiles);
+            const int64_t cost = ((wgs + slots - 1) / slots) * (tiles + kStartStages);
+            if (best < 0 || cost < best) {
+                best = cost;
+                p.tiles_per_wg = tiles;
+            }
+        }
+    }
     // grid.x * 256 work-items must stay below 2^32
     if ((int64_t)B * p.tgroups >= (1 << 24)) return fail(-1, "too many query groups (B * ceil(SQ * HI / 256))");
     const int rc = dsa::launch_indexer_logits(p, stream);

@@ -77,6 +77,11 @@ __device__ __forceinline__ float sum_xor32(float v) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// max(v, 0) (NaN becomes 0) in one instruction, the median of v, 0 and +inf:
+// fmaxf on an MFMA result costs a second one that quiets it first.  `inf` is
+// +inf in an opaque SGPR (a literal would be folded back into fmaxf).
+__device__ __forceinline__ float relu(float v, float inf) { return __builtin_amdgcn_fmed3f(v, 0.f, inf); }
+
 // One 1 KiB slice of a key tile (4 key rows x 256 B) straight into LDS: lane
 // l lands at m0 + 16 l, i.e. row l / 16, physical chunk l % 16, and loads the
 // logical chunk (l % 16) ^ (row % 16) of that row, so the B-fragment reads
@@ -100,8 +105,16 @@ __device__ __forceinline__ void load_slice(uint32_t lds_dst, rsrc_t rsrc, uint32
 // KS wave groups split every key stage (KS x 64 keys) and the workgroup's
 // 4 / KS query slots (64 query heads each) share it: KS = 1 for prefill (4
 // slots reuse each key tile), 2 or 4 when SQ is too small to fill the slots.
+//
+// Bound by the matrix cores in prefill: per 64 keys a wave issues 32 MFMAs (1024
+// cycles) and, for the head sum, two VALU instructions per product (512
+// cycles), which the SIMD's other wave hides (at most 256 registers a wave, so
+// that two fit and none of the products sits in an AGPR the VALU cannot read).
+// 4096 queries of 64 heads over 32768 keys: 1,646 us (1.25 PFLOP/s, what a large
+// library product reaches here) against 1,896 us with four instructions per
+// product; three waves per SIMD with the key blocks in sequence 1,730 us.
 template <int HI, int KS>
-__global__ __launch_bounds__(256, 1) void indexer_logits_kernel(IndexerParams p) {
+__global__ __launch_bounds__(256, KS == 4 ? 1 : 2) void indexer_logits_kernel(IndexerParams p) {
     static_assert(HI == 32 || HI == 64, "indexer heads");
     static_assert(KS == 1 || KS == 2 || KS == 4, "key split");
     constexpr int TG = 256 / HI / KS;            // queries per workgroup
@@ -176,6 +189,8 @@ __global__ __launch_bounds__(256, 1) void indexer_logits_kernel(IndexerParams p)
     issue(tile_begin);
     wait_vmcnt<0>();  // Q, weights and the first stage: nothing the compiler waits for stays in the loop
 
+    float inf = INFINITY;
+    asm volatile("" : "+s"(inf));
     float res[2][2];  // [hb][key block] sums of the previous stage, stored one iteration late
     int prev = -1;
     for (int tile = tile_begin; tile < tile_end; ++tile) {
@@ -211,7 +226,7 @@ __global__ __launch_bounds__(256, 1) void indexer_logits_kernel(IndexerParams p)
             for (int kb = 0; kb < 2; ++kb) {
                 float sum = 0.f;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) sum = fmaf(wv[hb][r], fmaxf(acc[hb][kb][r], 0.f), sum);
+                for (int r = 0; r < 16; ++r) sum = fmaf(wv[hb][r], relu(acc[hb][kb][r], inf), sum);
                 res[hb][kb] = sum_xor32(sum);
             }
         if constexpr (HI == 64) {  // the query's 64 heads are this wave's two blocks
