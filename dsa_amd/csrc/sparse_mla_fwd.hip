@@ -375,6 +375,26 @@ __device__ __forceinline__ void store_indices(const IdxRegs<CAP>& r, uint32_t id
         lds_store<int>(idx_lds + 4 * ((int)threadIdx.x + i * kThreads), m.v[i]);
 }
 
+// Tiles up to the range's last valid slot (at least one), by every wave for
+// itself from the index cache.  The tiles behind hold masked slots only, which
+// contribute exactly nothing: the selection pads a row at its end and the row
+// bucketing moves every masked slot there, so a prompt's first tokens, with
+// fewer keys than slots, run the tiles they fill (300 fresh queries of 16 heads
+// with 1024 slots 21 us against 48 us).  Called once a wave's first gathers are
+// issued, or while it would wait for them; straight-line, since a branch here would make the compiler's wait counts
+// for the register-staged gathers behind it conservative.
+template <int BN, int CAP = DSA_IDX_CAP>
+__device__ __forceinline__ int live_tiles(uint32_t idx_lds, int lane, int nt) {
+    int last = 0;
+#pragma unroll
+    for (int i = 0; i < CAP / 256; ++i) {
+        const i32x4 v = lds_load<i32x4>(idx_lds + 1024 * i + 16 * lane);
+        const uint64_t b = __ballot(max(max(v[0], v[1]), max(v[2], v[3])) >= 0);
+        last = b ? 256 * i + 256 - 4 * __builtin_clzll(b) : last;
+    }
+    return min(nt, max(1, (last + BN - 1) / BN));
+}
+
 // Compaction of the workgroup's slots (threads 0..255 hold the masked cache
 // values of mask_indices): the valid entries, in slot order, go to the front
 // of the cache and the last tile is padded with -1, so masked slots cost no
@@ -1114,7 +1134,7 @@ __device__ __forceinline__ void merge_if_last(const FwdParams& p, const WgCoords
     if (group_count_in(p, c, flag_lds)) merge_group_cols<NCB>(p, c, head0, heads, hl, g, writes_ml, cb_lo);
 }
 
-template <int HW, int KW, bool FP8 = false>
+template <int HW, int KW, bool FP8 = false, bool TRIM = false>
 __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd_narrow(FwdParams p) {
     static_assert(HW * KW == kWaves, "narrow variant shape");
     using R = std::conditional_t<FP8, RingFp8<64>, Ring<64, 2>>;
@@ -1132,7 +1152,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd_narrow(FwdParams p
     const int g = lane >> 4;
     const int n16 = lane & 15;
 
-    const WgCoords c = wg_coords<kBN>(p);
+    WgCoords c = wg_coords<kBN>(p);
     const int head = c.hgi * (16 * HW) + hw * 16 + n16;  // this lane's head
     // QK k-step ks (ks < 16) gives k-group g the 16-byte chunk 16 g + ks of the
     // 512 latent dims (Q and K agree; a dot product does not depend on the
@@ -1207,6 +1227,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd_narrow(FwdParams p
     // issuing tile t + 2 into the stage it has just finished reading.
     constexpr bool kOwnRows = HW == 1 && !FP8;
     if (c.nt > 0) issue(0);
+    if constexpr (TRIM) c.nt = live_tiles<kBN>(idx_lds, lane, c.nt);
     wait_vmcnt<0>();  // Q and tile 0 (see the wide variant)
     if constexpr (kOwnRows)
         if (c.nt > 1) issue(1);
@@ -1535,7 +1556,7 @@ struct XpLds {
     static_assert(2 * kWaves * BM * 4 <= RING, "epilogue exchange fits the ring");
 };
 
-template <int HB, bool PROD>
+template <int HB, bool PROD, bool TRIM = false>
 __global__ __launch_bounds__(PROD ? 2 * kThreads : kThreads, 1) void sparse_mla_fwd_xp(FwdParams p) {
     using R = Ring<64, 2>;
     using X = XpLds<HB>;
@@ -1552,7 +1573,7 @@ __global__ __launch_bounds__(PROD ? 2 * kThreads : kThreads, 1) void sparse_mla_
     const int g = lane >> 4;
     const int n16 = lane & 15;
 
-    const WgCoords c = wg_coords<kBN>(p);
+    WgCoords c = wg_coords<kBN>(p);
     const int head0 = c.hgi * X::BM;
     IdxRegs<X::IDX_CAP> ids;
     if (!producer) ids = fetch_indices<kBN, X::IDX_CAP>(p, c);
@@ -1616,6 +1637,7 @@ __global__ __launch_bounds__(PROD ? 2 * kThreads : kThreads, 1) void sparse_mla_
         bool ref_set = pass == 1;  // pass 1 runs against the exact max (set at the vote)
         bool overflow = false;
         if (!PROD || producer) issue_tile<R>(p, gt, 0, R::stage(lds, 0), idx_lds, gw, lane);
+        if constexpr (TRIM) c.nt = live_tiles<kBN, X::IDX_CAP>(idx_lds, lane, c.nt);
         wait_vmcnt<0>();  // Q and tile 0
 
         for (int t = 0; t < c.nt; ++t) {
@@ -2004,7 +2026,7 @@ __device__ __forceinline__ void xs_store(uint32_t stage, int j, int lane, const 
     __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int HB>
+template <int HB, bool TRIM = false>
 __global__ __launch_bounds__(64 * XsLds<HB>::WAVES, 1) void sparse_mla_fwd_xs(FwdParams p) {
     using X = XsLds<HB>;
     constexpr int BN = X::BN;
@@ -2017,7 +2039,7 @@ __global__ __launch_bounds__(64 * XsLds<HB>::WAVES, 1) void sparse_mla_fwd_xs(Fw
     const int g = lane >> 4;
     const int n16 = lane & 15;
 
-    const WgCoords c = wg_coords<BN>(p);
+    WgCoords c = wg_coords<BN>(p);
     const int head0 = c.hgi * BM;
     const uint32_t idx_lds = lds + X::IDX_OFF;
     const uint32_t p_lds = lds + X::P_OFF;
@@ -2087,6 +2109,7 @@ __global__ __launch_bounds__(64 * XsLds<HB>::WAVES, 1) void sparse_mla_fwd_xs(Fw
         for (int pass = 0; pass < 2; ++pass) {
 #pragma unroll
             for (int i = 0; i < X::DEPTH; ++i) xs_load(p, kv, kr, i, c.nt, idx_lds, j, lane, rb[i]);
+            if constexpr (TRIM) c.nt = live_tiles<BN>(idx_lds, lane, c.nt);
             xs_store(X::stage(lds, 0), j, lane, rb[0]);
             xs_load(p, kv, kr, X::DEPTH, c.nt, idx_lds, j, lane, rb[0]);
             xs_store(X::stage(lds, 1), j, lane, rb[1]);
@@ -2120,6 +2143,7 @@ __global__ __launch_bounds__(64 * XsLds<HB>::WAVES, 1) void sparse_mla_fwd_xs(Fw
         return;
     }
 
+    if constexpr (TRIM) c.nt = live_tiles<BN>(idx_lds, lane, c.nt);
     if (wave < HB) {
         // ---- QK waves: S^T = K . Q^T for the tile's two 16-row subtiles.
         const int hb = wave;
@@ -2832,6 +2856,8 @@ __global__ __launch_bounds__(kPPThreads, 1) void sparse_mla_fwd_pp(FwdParams p) 
     }
 }
 
+constexpr int kTrimMinQueries = 32;  // queries per sequence from which a call is a chunk, not a decode step
+
 template <typename K>
 int launch(K kernel, const FwdParams& p, hipStream_t stream, int threads = kThreads) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)fwd_grid(p)), dim3(threads), 0, stream, p);
@@ -2868,13 +2894,21 @@ int fwd_index_cap(int hpg, int bn, int pv_cols) {
 int launch_fwd(const FwdParams& p, int hpg, int kvw, int bn, int stages, int mfma, int pv_cols, hipStream_t stream) {
     if (!fwd_variant_exists(hpg, kvw, bn, stages, mfma, pv_cols)) return (int)hipErrorInvalidValue;
     if (p.kv_fp8 && (mfma != 16 || pv_cols != 512)) return (int)hipErrorInvalidValue;  // fp8 rows: narrow variants only
+    // Chunks of one sequence's queries look for the last valid slot first (the
+    // ping-pong kernels compact in any case); decode calls, whose rows are full
+    // but for a short context, run the kernels without that step (it costs the
+    // 8-token decode 0.3 us of 21).
+    const bool trim = p.SQ >= kTrimMinQueries;
     if (pv_cols == 128) {
         if (hpg == 128) return launch(sparse_mla_fwd_pp<false>, p, stream, kPPThreads);
         if (hpg == 64 && bn == 32) return launch(sparse_mla_fwd_pp<true>, p, stream, kPPThreads);
-        if (hpg == 16 && bn == 32) return launch(sparse_mla_fwd_xs<1>, p, stream, 64 * XsLds<1>::WAVES);
-        if (hpg == 32 && bn == 32) return launch(sparse_mla_fwd_xs<2>, p, stream, 64 * XsLds<2>::WAVES);
-        if (hpg == 16) return launch(sparse_mla_fwd_xp<1, true>, p, stream, 2 * kThreads);
-        if (hpg == 32) return launch(sparse_mla_fwd_xp<2, false>, p, stream);
+        if (hpg == 16 && bn == 32)
+            return launch(trim ? sparse_mla_fwd_xs<1, true> : sparse_mla_fwd_xs<1>, p, stream, 64 * XsLds<1>::WAVES);
+        if (hpg == 32 && bn == 32)
+            return launch(trim ? sparse_mla_fwd_xs<2, true> : sparse_mla_fwd_xs<2>, p, stream, 64 * XsLds<2>::WAVES);
+        if (hpg == 16)
+            return launch(trim ? sparse_mla_fwd_xp<1, true, true> : sparse_mla_fwd_xp<1, true>, p, stream, 2 * kThreads);
+        if (hpg == 32) return launch(trim ? sparse_mla_fwd_xp<2, false, true> : sparse_mla_fwd_xp<2, false>, p, stream);
         return launch(sparse_mla_fwd_xp<4, false>, p, stream);
     }
     if (mfma == 32) {
@@ -2882,9 +2916,11 @@ int launch_fwd(const FwdParams& p, int hpg, int kvw, int bn, int stages, int mfm
         return launch(sparse_mla_fwd_wide<2, 2, 64, 2>, p, stream);
     }
     if (p.kv_fp8) {
-        if (hpg == 64) return launch(sparse_mla_fwd_narrow<4, 1, true>, p, stream);
-        if (hpg == 32) return launch(sparse_mla_fwd_narrow<2, 2, true>, p, stream);
-        return launch(sparse_mla_fwd_narrow<1, 4, true>, p, stream);
+        if (hpg == 64)
+            return launch(trim ? sparse_mla_fwd_narrow<4, 1, true, true> : sparse_mla_fwd_narrow<4, 1, true>, p, stream);
+        if (hpg == 32)
+            return launch(trim ? sparse_mla_fwd_narrow<2, 2, true, true> : sparse_mla_fwd_narrow<2, 2, true>, p, stream);
+        return launch(trim ? sparse_mla_fwd_narrow<1, 4, true, true> : sparse_mla_fwd_narrow<1, 4, true>, p, stream);
     }
     if (hpg == 64) return launch(sparse_mla_fwd_narrow<4, 1>, p, stream);
     if (hpg == 32) return launch(sparse_mla_fwd_narrow<2, 2>, p, stream);
