@@ -322,14 +322,17 @@ def project_uv(output, w_uv):
     dv, head_stride = _check_w_uv(w_uv, heads, device)
     tokens = output.numel() // (heads * HEAD_DIM)
     out_v = torch.empty((*output.shape[:-1], dv), device=device, dtype=torch.bfloat16)
-    if tokens == 0:
-        return out_v
-    stream = torch.cuda.current_stream(device).cuda_stream
-    with torch.cuda.device(device):
-        rc = _lib.load().dsa_project_uv(_vp(output), _vp(w_uv), head_stride, _vp(out_v), tokens, heads, dv,
-                                        ctypes.c_void_p(stream))
-    _lib.check(rc, "dsa_project_uv")
+    if tokens > 0:
+        stream = torch._C._cuda_getCurrentRawStream(device.index)
+        _project_uv_into(out_v, output, w_uv, head_stride, tokens, heads, dv, stream)
     return out_v
+
+
+def _project_uv_into(out_v, output, w_uv, head_stride, tokens, heads, dv, stream):
+    with _on_device(output.device):
+        rc = _lib.load().dsa_project_uv(output.data_ptr(), w_uv.data_ptr(), head_stride, out_v.data_ptr(), tokens,
+                                        heads, dv, stream)
+    _lib.check(rc, "dsa_project_uv")
 
 
 def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_kernels=False,
@@ -408,31 +411,43 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
     config, partials, launches, plan, fused, groups = _call_plan(shape, config, cores, fp8, uv_dim)
     if fused and arrivals is not None and arrivals.numel() < groups:
         raise ValueError(f"arrivals holds {arrivals.numel()} counters; this call needs {groups}")
-    expanded = None
-    if fp8 and default_plan and arrivals is None and expands_rows(shape):
-        expanded = _expanded_cache(kv, block_table, shape)
-        if expanded is not None:
-            config, partials, launches, plan, fused, groups = _call_plan(shape, None, cores, False, uv_dim)
-            launches = (Launch("expand_rows", _expand_grid(batch * length), 256, 0),) + launches
     bucket = buckets_rows(shape)
     if (default_plan and cores == _device_cus(device) and not fused and not fp8 and scale is None
             and block_table is None and uv is None and not bucket):
         _register_fast(device, shape, plan, partials)
 
+    stream = torch._C._cuda_getCurrentRawStream(device.index)
     output = torch.empty_like(q)
     maximum = torch.empty((batch, 1, queries, heads), device=device, dtype=torch.float32)
     denominator = torch.empty_like(maximum)
-    if partials is None:
-        part_o = part_m = part_l = None
-    else:
+    out_v = None if uv is None else torch.empty((batch, queries, heads, uv[0]), device=device, dtype=torch.bfloat16)
+    order = torch.empty_like(indices) if bucket else None
+    # The expanded cache after every buffer that the call needs in any case, and
+    # given up if the buffers of the plan that reads it do not fit beside it: a
+    # call that fits on the fp8 rows never fails for the expansion's sake.
+    expanded = work = None
+    if fp8 and default_plan and arrivals is None and expands_rows(shape):
+        expanded = _expanded_cache(kv, block_table, shape)
+        if expanded is not None:
+            bf16 = _call_plan(shape, None, cores, False, uv_dim)
+            try:
+                work = _work_buffers(bf16, arrivals, device, stream)
+            except torch.OutOfMemoryError:
+                expanded = None
+            else:
+                config, partials, launches, plan, fused, groups = bf16
+                launches = (Launch("expand_rows", _expand_grid(batch * length), 256, 0),) + launches
+    if work is None:
+        work = _work_buffers((config, partials, launches, plan, fused, groups), arrivals, device, stream)
+    part_buf, counters = work
+    part_o = part_m = part_l = None
+    if part_buf is not None:
         # One buffer carved into part_o, part_m, part_l (each 256-byte aligned):
         # only their addresses leave this function.
-        part_buf = torch.empty(partials[2], device=device, dtype=torch.float32)
         part_o = part_buf.data_ptr()
         part_m = part_o + partials[3]
         part_l = part_o + partials[4]
 
-    stream = torch._C._cuda_getCurrentRawStream(device.index)
     lib = _lib.load()
     idx_ptr = indices.data_ptr()
     kv_ptr, rope_ptr = kv.data_ptr(), None if k_rope is None else k_rope.data_ptr()
@@ -447,7 +462,6 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
             _lib.check(rc, "dsa_kv_expand_rows")
         kv_ptr, rope_ptr = expanded.data_ptr(), expanded.data_ptr() + rope_row
     if bucket:
-        order = torch.empty_like(indices)
         with _on_device(device):
             if expanded is not None and block_table is not None:
                 rc = lib.dsa_bucket_indices_paged(idx_ptr, order.data_ptr(), batch, queries, topk, length, *pages,
@@ -473,7 +487,6 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
         else:
             opts = _options(scale, fp8, kv, block_table)
             if fused:
-                counters = arrivals if arrivals is not None else _arrival_counters(device, stream, groups)
                 opts.arrivals = counters.data_ptr()
             rc = lib.dsa_fwd_opts(*args, ctypes.byref(opts), plan, stream)
     if rc:
@@ -482,7 +495,6 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
         result = (output, maximum, denominator)
     elif merge_uv:
         dv, head_stride = uv
-        out_v = torch.empty((batch, queries, heads, dv), device=device, dtype=torch.bfloat16)
         with _on_device(device):
             rc = lib.dsa_merge_uv(part_o, part_m, part_l, w_uv.data_ptr(), head_stride, out_v.data_ptr(),
                                   maximum.data_ptr(), denominator.data_ptr(), batch * queries, heads,
@@ -490,10 +502,21 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
         _lib.check(rc, "dsa_merge_uv")
         result = (out_v, maximum, denominator)
     else:
-        result = (project_uv(output, w_uv), maximum, denominator)
+        _project_uv_into(out_v, output, w_uv, uv[1], batch * queries, heads, uv[0], stream)
+        result = (out_v, maximum, denominator)
     if return_kernels:
         return result, launches
     return result
+
+
+def _work_buffers(call, arrivals, device, stream):
+    """The partials of a split plan and the arrival counters of a fused one,
+    None where the plan (a _call_plan result) needs none."""
+    _, partials, _, _, fused, groups = call
+    part_buf = None if partials is None else torch.empty(partials[2], device=device, dtype=torch.float32)
+    if not fused:
+        return part_buf, None
+    return part_buf, arrivals if arrivals is not None else _arrival_counters(device, stream, groups)
 
 
 def _expanded_cache(kv, block_table, shape):

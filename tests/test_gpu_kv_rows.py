@@ -5,6 +5,8 @@ those of the tensor code (run on the same GPU tensors) for every bf16 block
 maximum, zeros, infinities and NaNs included, at row counts around a wave's
 pair of rows and the grid's reach, and for strided and misaligned views.
 """
+import weakref
+
 import pytest
 import torch
 
@@ -148,3 +150,65 @@ def test_call_without_room_runs_on_the_rows(monkeypatch):
     assert all(l.name != "expand_rows" for l in launches)
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+class _BudgetTorch:
+    """``torch`` whose ``empty``/``empty_like``/``zeros`` raise OutOfMemoryError
+    beyond ``budget`` live bytes (an idealised card; the tensors are real)."""
+
+    def __init__(self, budget):
+        self.budget, self.live, self.peak = budget, 0, 0
+
+    def __getattr__(self, name):
+        attr = getattr(torch, name)
+        if name not in ("empty", "empty_like", "zeros"):
+            return attr
+
+        def allocate(*args, **kwargs):
+            t = attr(*args, **kwargs)
+            size = t.numel() * t.element_size()
+            if self.live + size > self.budget:
+                del t
+                raise torch.OutOfMemoryError("beyond the test's budget")
+            self.live += size
+            self.peak = max(self.peak, self.live)
+            weakref.finalize(t, self._free, size)
+            return t
+        return allocate
+
+    def _free(self, size):
+        self.live -= size
+
+
+@pytest.mark.parametrize("shape,value_dim", [((1, 300, 96, 1024, 4096), 0),     # the bf16 plan splits too
+                                             ((1, 300, 96, 1024, 4096), 128),   # ... merge and projection in one
+                                             ((1, 257, 128, 1024, 257), 128)])  # no split, projected afterwards
+def test_expansion_never_takes_a_buffer_the_call_needs(monkeypatch, shape, value_dim):
+    """With any memory from what the call needs on the fp8 rows upwards it
+    succeeds: expanded where everything fits beside the cache, else on the rows."""
+    from dsa_amd import api
+
+    q, qr, ids, rows, _, _ = _expanding_case(*shape, 0, seed=6)
+    args = (q.cuda(), rows.cuda(), qr.cuda(), None, ids.cuda())
+    kw = {"w_uv": torch.randn(shape[2], value_dim, 512).bfloat16().cuda() * 0.04} if value_dim else {}
+
+    def run(budget, room=True, **more):
+        api._arrivals.clear()
+        spy = _BudgetTorch(budget)
+        with monkeypatch.context() as m:
+            m.setattr(api, "torch", spy)
+            if not room:
+                m.setattr(api, "_expanded_cache", lambda *_: None)
+            out, launches = dsa_amd.forward(*args, return_kernels=True, **kw, **more)
+        return out, launches[0].name == "expand_rows", spy.peak
+
+    on_rows, expanded, need = run(1 << 40, room=False)
+    assert not expanded
+    as_bf16, expanded, full = run(1 << 40)
+    assert expanded and full >= need
+    cache = shape[0] * shape[3] * 1152
+    for budget in (need, need + cache // 2, need + cache - 1, full - 1, full):
+        out, expanded, _ = run(budget)
+        assert expanded == (budget >= full), (budget, need, full)
+        for a, b in zip(out, as_bf16 if expanded else on_rows):
+            assert torch.equal(a, b)
