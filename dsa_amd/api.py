@@ -525,10 +525,29 @@ def _expanded_cache(kv, block_table, shape):
     itself then says so) or the memory is not there (it runs on the fp8 rows)."""
     if block_table is not None and kv.shape[0] * kv.shape[1] >= 1 << 25:
         return None
+    elems = shape[0] * shape[3] * (HEAD_DIM + ROPE_DIM)
+    if not _has_room(2 * elems, kv.device):
+        return None
     try:
-        return torch.empty(shape[0] * shape[3] * (HEAD_DIM + ROPE_DIM), device=kv.device, dtype=torch.bfloat16)
+        return torch.empty(elems, device=kv.device, dtype=torch.bfloat16)
     except torch.OutOfMemoryError:
         return None
+
+
+def _has_room(size: int, device) -> bool:
+    """Whether ``size`` bytes can be had on the device: free there and within the
+    process's memory fraction, or together with the cached blocks that torch's
+    allocator could give back.  Where not, asking the allocator would make it
+    wait for the device and empty its cache before it fails, on every call.
+    (10 us of host time; while capturing, the allocator keeps its cache.)"""
+    if torch.cuda.is_current_stream_capturing():
+        return True
+    free, total = torch.cuda.mem_get_info(device)
+    stats = torch._C._cuda_memoryStats(device.index)
+    now = lambda name: stats[name]["all"]["current"]  # noqa: E731
+    reserved = now("reserved_bytes")
+    allowed = int(total * torch.cuda.get_per_process_memory_fraction(device)) - reserved
+    return min(free, allowed) + reserved - now("active_bytes") - now("inactive_split_bytes") >= size
 
 
 def _expand_grid(rows: int) -> int:

@@ -212,3 +212,34 @@ def test_expansion_never_takes_a_buffer_the_call_needs(monkeypatch, shape, value
         assert expanded == (budget >= full), (budget, need, full)
         for a, b in zip(out, as_bf16 if expanded else on_rows):
             assert torch.equal(a, b)
+
+
+def test_call_without_room_keeps_the_allocators_cache():
+    """Where the copy cannot be had, torch's allocator is not asked for it: it
+    would wait for the device and give every cached block back first."""
+    shape = (1, 512, 16, 65536, 2048)  # a copy of 72 MiB
+    q, qr, ids, rows, _, _ = _expanding_case(*shape, 0, seed=2)
+    args = (q.cuda(), rows.cuda(), qr.cuda(), None, ids.cuda())
+    want = dsa_amd.forward(*args, config=dsa_amd.plan_call(shape, None, 256, kv_fp8=True)[0])
+    got, launches = dsa_amd.forward(*args, return_kernels=True)
+    assert launches[0].name == "expand_rows"
+    del got
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    kept = torch.empty(16 << 20, device="cuda", dtype=torch.uint8)
+    del kept  # a cached block
+    room = 40 << 20  # the call's own buffers and no copy
+    total = torch.cuda.mem_get_info()[1]
+    before = torch.cuda.get_per_process_memory_fraction()
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + room) / total)
+    try:
+        retries = torch.cuda.memory_stats()["num_alloc_retries"]
+        for _ in range(2):
+            got, launches = dsa_amd.forward(*args, return_kernels=True)
+            assert launches[0].name != "expand_rows"
+            for a, b in zip(got, want):
+                assert torch.equal(a, b)
+            del got
+        assert torch.cuda.memory_stats()["num_alloc_retries"] == retries
+    finally:
+        torch.cuda.set_per_process_memory_fraction(before)
