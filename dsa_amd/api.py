@@ -370,7 +370,9 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
     with ``bf16(fp32(e4m3) * scale)`` latent values.  A prefill-sized call
     without a ``config`` that gathers each cache row often (:func:`expands_rows`)
     first writes those values into a buffer of its own and then runs as a bf16
-    call: the same values through other kernels.
+    call: the same values through other kernels.  Where there is no room for
+    that buffer (up to 1 GiB), or ``arrivals`` holds enough counters for the
+    plan on the fp8 rows but not for the bf16 plan, it runs on the fp8 rows.
 
     ``w_uv`` (bf16 ``[H, dv, 512]``, dv a multiple of 64 up to 256; heads may
     be any stride apart, so ``wkv_b.view(H, d_nope + dv, 512)[:, -dv:]`` goes
@@ -426,10 +428,11 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
     # given up if the buffers of the plan that reads it do not fit beside it: a
     # call that fits on the fp8 rows never fails for the expansion's sake.
     expanded = work = None
-    if fp8 and default_plan and arrivals is None and expands_rows(shape):
-        expanded = _expanded_cache(kv, block_table, shape)
+    if fp8 and default_plan and expands_rows(shape):
+        bf16 = _call_plan(shape, None, cores, False, uv_dim)
+        few = bf16[4] and arrivals is not None and arrivals.numel() < bf16[5]  # counters of the fp8 plan's size
+        expanded = None if few else _expanded_cache(kv, block_table, shape)
         if expanded is not None:
-            bf16 = _call_plan(shape, None, cores, False, uv_dim)
             try:
                 work = _work_buffers(bf16, arrivals, device, stream)
             except torch.OutOfMemoryError:

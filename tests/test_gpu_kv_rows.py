@@ -243,3 +243,37 @@ def test_call_without_room_keeps_the_allocators_cache():
         assert torch.cuda.memory_stats()["num_alloc_retries"] == retries
     finally:
         torch.cuda.set_per_process_memory_fraction(before)
+
+
+@pytest.mark.parametrize("shape", [(1, 300, 128, 1024, 512),    # neither plan fuses its merge
+                                   (1, 257, 16, 1024, 4096)])   # both do, one counter a token
+def test_expansion_does_not_depend_on_arrivals(shape):
+    """The caller's own counters change nothing but whose counters are used."""
+    q, qr, ids, rows, _, _ = _expanding_case(*shape, 0, seed=8)
+    args = (q.cuda(), rows.cuda(), qr.cuda(), None, ids.cuda())
+    want, launches = dsa_amd.forward(*args, return_kernels=True)
+    own = torch.zeros(shape[0] * shape[1] * shape[2] // 16, device="cuda", dtype=torch.int32)
+    got, with_own = dsa_amd.forward(*args, return_kernels=True, arrivals=own)
+    assert with_own == launches and launches[0].name == "expand_rows"
+    torch.cuda.synchronize()
+    assert not own.any()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+def test_counters_of_the_fp8_plans_size_are_taken():
+    """Enough counters for the plan on the fp8 rows (32 heads a workgroup), too
+    few for the bf16 plan (16 heads): such a call runs on the fp8 rows."""
+    shape = (1, 256, 32, 1024, 4096)
+    on_rows, as_bf16 = dsa_amd.plan_call(shape, kv_fp8=True)[0], dsa_amd.plan_call(shape)[0]
+    assert on_rows.fused_merge and as_bf16.fused_merge and on_rows.bm > as_bf16.bm
+    q, qr, ids, rows, _, _ = _expanding_case(*shape, 0, seed=10)
+    args = (q.cuda(), rows.cuda(), qr.cuda(), None, ids.cuda())
+    want = dsa_amd.forward(*args, config=on_rows)
+    own = torch.zeros(shape[0] * shape[1] * shape[2] // on_rows.bm, device="cuda", dtype=torch.int32)
+    got, launches = dsa_amd.forward(*args, return_kernels=True, arrivals=own)
+    assert launches[0].name != "expand_rows"
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    with pytest.raises(ValueError, match="counters"):
+        dsa_amd.forward(*args, arrivals=own[1:])
