@@ -110,6 +110,11 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+def built() -> bool:
+    """Whether :func:`load` has a library to load (or has loaded it)."""
+    return _lib is not None or LIB_PATH.exists()
+
+
 def last_error() -> str:
     return load().dsa_last_error().decode(errors="replace")
 

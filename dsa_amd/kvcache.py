@@ -55,8 +55,9 @@ def quantize_kv_fp8(kv, k_rope, pow2_scales: bool = True):
 def _plain_gpu_pair(kv, k_rope):
     """Whether the kernel may read these two tensors: ordinary eager tensors
     of one ROCm GPU (no subclass, tracing, dispatch mode or functorch level
-    between the caller and the storage) with at least one row."""
-    return (type(kv) is torch.Tensor and type(k_rope) is torch.Tensor and kv.is_cuda and kv.device == k_rope.device
+    between the caller and the storage) with at least one row, and the library
+    built (the rows can be written without it, unlike the attention's results)."""
+    return (_lib.built() and type(kv) is torch.Tensor and type(k_rope) is torch.Tensor and kv.is_cuda and kv.device == k_rope.device
             and torch.version.hip is not None and kv.numel() > 0 and not torch.compiler.is_compiling()
             and not torch.jit.is_tracing() and not torch._C._are_functorch_transforms_active()
             and torch._C._len_torch_dispatch_stack() == 0 and not (kv.is_neg() or k_rope.is_neg()))

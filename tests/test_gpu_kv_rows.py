@@ -68,6 +68,18 @@ def test_row_counts(monkeypatch, rows, pow2):
         assert torch.equal(out.cpu(), dsa_amd.quantize_kv_fp8(kv, kr))
 
 
+def test_rows_without_the_library(monkeypatch, tmp_path):
+    """A package whose library is not built writes the rows as tensor code."""
+    from dsa_amd import _lib
+
+    g = torch.Generator().manual_seed(12)
+    kv, kr = torch.randn(5, 512, generator=g).bfloat16().cuda(), torch.randn(5, 64, generator=g).bfloat16().cuda()
+    want = _launched(monkeypatch, kv, kr)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "missing.so")
+    assert torch.equal(dsa_amd.quantize_kv_fp8(kv, kr), want)
+
+
 def test_views(monkeypatch):
     g = torch.Generator().manual_seed(3)
     both = torch.randn(6, 577 + 3, generator=g).bfloat16().cuda()
