@@ -21,6 +21,8 @@ ones) by the same arithmetic as tensor code, to the same bytes.
 from __future__ import annotations
 
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from .api import _on_device
@@ -54,13 +56,21 @@ def quantize_kv_fp8(kv, k_rope, pow2_scales: bool = True):
 
 def _plain_gpu_pair(kv, k_rope):
     """Whether the kernel may read these two tensors: ordinary eager tensors
-    of one ROCm GPU (no subclass, tracing, dispatch mode or functorch level
+    of one ROCm GPU (no subclass, tracing, function or dispatch mode or functorch level
     between the caller and the storage) with at least one row, and the library
     built (the rows can be written without it, unlike the attention's results)."""
     return (_lib.built() and type(kv) is torch.Tensor and type(k_rope) is torch.Tensor and kv.is_cuda and kv.device == k_rope.device
             and torch.version.hip is not None and kv.numel() > 0 and not torch.compiler.is_compiling()
             and not torch.jit.is_tracing() and not torch._C._are_functorch_transforms_active()
-            and torch._C._len_torch_dispatch_stack() == 0 and not (kv.is_neg() or k_rope.is_neg()))
+            and torch._C._len_torch_dispatch_stack() == 0 and not _function_modes() and not (kv.is_neg() or k_rope.is_neg()))
+
+
+def _function_modes() -> bool:
+    """Whether a torch_function mode watches the operations.  A default device
+    (``torch.set_default_device``) is such a mode too, but only places tensors
+    that name no device."""
+    return (torch._C._len_torch_function_stack() > 0
+            and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
 
 
 def _quantize_gpu(kv, k_rope, lead, pow2_scales):

@@ -68,6 +68,28 @@ def test_row_counts(monkeypatch, rows, pow2):
         assert torch.equal(out.cpu(), dsa_amd.quantize_kv_fp8(kv, kr))
 
 
+def test_function_modes_see_the_operations(monkeypatch):
+    """A torch_function mode sees every operation of the row writer, as of any
+    tensor code; a default device is no such observer."""
+    from torch.overrides import TorchFunctionMode
+
+    seen = []
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", str(func)))
+            return func(*args, **(kwargs or {}))
+
+    g = torch.Generator().manual_seed(13)
+    kv, kr = torch.randn(5, 512, generator=g).bfloat16().cuda(), torch.randn(5, 64, generator=g).bfloat16().cuda()
+    want = _launched(monkeypatch, kv, kr)
+    with Watch():
+        rows = dsa_amd.quantize_kv_fp8(kv, kr)
+    assert torch.equal(rows, want) and {"float", "where", "frexp", "cat"} <= set(seen)
+    with torch.device("cpu"):
+        assert torch.equal(_launched(monkeypatch, kv, kr), want)
+
+
 def test_rows_without_the_library(monkeypatch, tmp_path):
     """A package whose library is not built writes the rows as tensor code."""
     from dsa_amd import _lib
