@@ -384,24 +384,33 @@ __device__ __forceinline__ void store_indices(const IdxRegs<CAP>& r, uint32_t id
         lds_store<int>(idx_lds + 4 * ((int)threadIdx.x + i * kThreads), m.v[i]);
 }
 
+// The range's last index (a scalar load beside the index loads; every wave reads
+// the same word).  A range that ends in a valid slot has no tiles to leave out,
+// and live_tiles is not run for it.
+__device__ __forceinline__ int last_index(const FwdParams& p, const WgCoords& c, int bn) {
+    const int last = min(c.slot0 + c.nt * bn, p.TOPK) - 1;
+    return p.idx[(int64_t)c.token * p.TOPK + max(last, 0)];
+}
+__device__ __forceinline__ bool masked_index(const FwdParams& p, int id) {
+    id = __builtin_amdgcn_readfirstlane(id);
+    asm volatile("" : "+s"(id));  // waited for here, ahead of the barrier behind the index loads
+    return __builtin_expect((uint32_t)id >= (uint32_t)p.L, 0);
+}
+
 // Tiles up to the range's last valid slot (at least one), by every wave for
 // itself from the index cache.  The tiles behind hold masked slots only, which
 // contribute exactly nothing: the selection pads a row at its end and the row
 // bucketing moves every masked slot there, so a prompt's first tokens, with
 // fewer keys than slots, run the tiles they fill (300 fresh queries of 16 heads
-// with 1024 slots 21 us against 48 us).  Called once a wave's first gathers are
-// issued, or while it would wait for them; straight-line, since a branch here would make the compiler's wait counts
-// for the register-staged gathers behind it conservative.
-template <int BN, int CAP = DSA_IDX_CAP>
+// with 1024 slots 21 us against 48 us).
+template <int BN>
 __device__ __forceinline__ int live_tiles(uint32_t idx_lds, int lane, int nt) {
-    int last = 0;
-#pragma unroll
-    for (int i = 0; i < CAP / 256; ++i) {
+    for (int i = (nt * BN + 255) / 256 - 1; i >= 0; --i) {
         const i32x4 v = lds_load<i32x4>(idx_lds + 1024 * i + 16 * lane);
         const uint64_t b = __ballot(max(max(v[0], v[1]), max(v[2], v[3])) >= 0);
-        last = b ? 256 * i + 256 - 4 * __builtin_clzll(b) : last;
+        if (b) return min(nt, (256 * i + 256 - 4 * __builtin_clzll(b) + BN - 1) / BN);
     }
-    return min(nt, max(1, (last + BN - 1) / BN));
+    return min(nt, 1);
 }
 
 // Compaction of the workgroup's slots (threads 0..255 hold the masked cache
@@ -1162,6 +1171,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd_narrow(FwdParams p
     const int n16 = lane & 15;
 
     WgCoords c = wg_coords<kBN>(p);
+    const int last = TRIM ? last_index(p, c, kBN) : 0;
     const int head = c.hgi * (16 * HW) + hw * 16 + n16;  // this lane's head
     // QK k-step ks (ks < 16) gives k-group g the 16-byte chunk 16 g + ks of the
     // 512 latent dims (Q and K agree; a dot product does not depend on the
@@ -1190,6 +1200,7 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd_narrow(FwdParams p
 
     const uint32_t idx_lds = lds + R::IDX_OFF;
     store_indices<kBN>(ids, idx_lds, p, c);
+    const bool tail = TRIM && masked_index(p, last);
     lds_barrier();
     const Gather gt = make_gather(p, c.b);
     const char* fp8_rows = fp8_base(p, c.b);
@@ -1236,11 +1247,15 @@ __global__ __launch_bounds__(kThreads, 1) void sparse_mla_fwd_narrow(FwdParams p
     // issuing tile t + 2 into the stage it has just finished reading.
     constexpr bool kOwnRows = HW == 1 && !FP8;
     if (c.nt > 0) issue(0);
-    if constexpr (TRIM) c.nt = live_tiles<kBN>(idx_lds, lane, c.nt);
+    if constexpr (TRIM)
+        if (__builtin_expect(tail, 0)) c.nt = live_tiles<kBN>(idx_lds, lane, c.nt);
     wait_vmcnt<0>();  // Q and tile 0 (see the wide variant)
     if constexpr (kOwnRows)
         if (c.nt > 1) issue(1);
 
+    // The loop 8 bytes behind a 32-byte boundary: 200 queries of 16 heads over
+    // fp8 rows 128.5 us here, 130 to 133 us further behind.
+    if constexpr (TRIM) asm volatile(".p2align 5\n\t.rept 2\n\ts_nop 0\n\t.endr");
     for (int t = 0; t < c.nt; ++t) {
         if constexpr (kOwnRows) {
             if (t > 0) {  // tile t has landed; tile t + 1 may stay in flight
@@ -1583,6 +1598,7 @@ __global__ __launch_bounds__(PROD ? 2 * kThreads : kThreads, 1) void sparse_mla_
     const int n16 = lane & 15;
 
     WgCoords c = wg_coords<kBN>(p);
+    const int last = TRIM ? last_index(p, c, kBN) : 0;
     const int head0 = c.hgi * X::BM;
     IdxRegs<X::IDX_CAP> ids;
     if (!producer) ids = fetch_indices<kBN, X::IDX_CAP>(p, c);
@@ -1603,6 +1619,7 @@ __global__ __launch_bounds__(PROD ? 2 * kThreads : kThreads, 1) void sparse_mla_
 
     const uint32_t idx_lds = lds + X::IDX_OFF;
     if (!producer) store_indices<kBN>(ids, idx_lds, p, c);
+    const bool tail = TRIM && masked_index(p, last);
     lds_barrier();
     const Gather gt = make_gather(p, c.b);
 
@@ -1646,7 +1663,8 @@ __global__ __launch_bounds__(PROD ? 2 * kThreads : kThreads, 1) void sparse_mla_
         bool ref_set = pass == 1;  // pass 1 runs against the exact max (set at the vote)
         bool overflow = false;
         if (!PROD || producer) issue_tile<R>(p, gt, 0, R::stage(lds, 0), idx_lds, gw, lane);
-        if constexpr (TRIM) c.nt = live_tiles<kBN, X::IDX_CAP>(idx_lds, lane, c.nt);
+        if constexpr (TRIM)
+        if (__builtin_expect(tail, 0)) c.nt = live_tiles<kBN>(idx_lds, lane, c.nt);
         wait_vmcnt<0>();  // Q and tile 0
 
         for (int t = 0; t < c.nt; ++t) {
@@ -2049,6 +2067,7 @@ __global__ __launch_bounds__(64 * XsLds<HB>::WAVES, 1) void sparse_mla_fwd_xs(Fw
     const int n16 = lane & 15;
 
     WgCoords c = wg_coords<BN, true>(p);
+    const int last = TRIM ? last_index(p, c, BN) : 0;
     const int head0 = c.hgi * BM;
     const uint32_t idx_lds = lds + X::IDX_OFF;
     const uint32_t p_lds = lds + X::P_OFF;
@@ -2071,6 +2090,7 @@ __global__ __launch_bounds__(64 * XsLds<HB>::WAVES, 1) void sparse_mla_fwd_xs(Fw
         qf[16] = *reinterpret_cast<const bf16x8*>(rrow);
         qf[17] = *reinterpret_cast<const bf16x8*>(rrow + 32);
     }
+    const bool tail = TRIM && masked_index(p, last);
     lds_barrier();
 
     // Second-pass vote (every wave): the flag is raised by a QK wave whose
@@ -2114,11 +2134,13 @@ __global__ __launch_bounds__(64 * XsLds<HB>::WAVES, 1) void sparse_mla_fwd_xs(Fw
         const char* kv = reinterpret_cast<const char*>(p.kv) + first * 1024;
         const char* kr = reinterpret_cast<const char*>(p.k_rope) + first * 128;
         XsRows rb[X::DEPTH];
+        // ahead of the loads: a branch behind them would make the compiler's wait counts conservative
+        if constexpr (TRIM)
+            if (__builtin_expect(tail, 0)) c.nt = live_tiles<BN>(idx_lds, lane, c.nt);
 #pragma unroll 1
         for (int pass = 0; pass < 2; ++pass) {
 #pragma unroll
             for (int i = 0; i < X::DEPTH; ++i) xs_load(p, kv, kr, i, c.nt, idx_lds, j, lane, rb[i]);
-            if constexpr (TRIM) c.nt = live_tiles<BN>(idx_lds, lane, c.nt);
             xs_store(X::stage(lds, 0), j, lane, rb[0]);
             xs_load(p, kv, kr, X::DEPTH, c.nt, idx_lds, j, lane, rb[0]);
             xs_store(X::stage(lds, 1), j, lane, rb[1]);
@@ -2152,7 +2174,8 @@ __global__ __launch_bounds__(64 * XsLds<HB>::WAVES, 1) void sparse_mla_fwd_xs(Fw
         return;
     }
 
-    if constexpr (TRIM) c.nt = live_tiles<BN>(idx_lds, lane, c.nt);
+    if constexpr (TRIM)
+        if (__builtin_expect(tail, 0)) c.nt = live_tiles<BN>(idx_lds, lane, c.nt);
     if (wave < HB) {
         // ---- QK waves: S^T = K . Q^T for the tile's two 16-row subtiles.
         const int hb = wave;
@@ -2162,6 +2185,10 @@ __global__ __launch_bounds__(64 * XsLds<HB>::WAVES, 1) void sparse_mla_fwd_xs(Fw
             l_run = 0.f;
             if (pass == 1) m_ref = m_true;  // pass 1 runs against the exact max
             bool overflow = false;
+            // The loop's head 16 bytes into a fetch window of 32: the QK waves set
+            // the pace and run up to 2.5 % slower from other offsets (1500 queries
+            // of 96 heads 986 us here, 990 to 1,012 us at the others).
+            if constexpr (TRIM) asm volatile(".p2align 5\n\t.rept 5\n\ts_nop 0\n\t.endr");
             for (int s = 0; s <= c.nt; ++s) {
                 lds_barrier();
                 if (s == c.nt) break;

@@ -86,3 +86,33 @@ def test_split_ranges_without_a_valid_slot(plan):
     # max of its query's heads, not element by element.
     assert O.accuracy(mx, ref[1])["max_row_normalized"] <= STAT_RTOL
     assert O.rel_error(sm, ref[2]) <= STAT_RTOL
+
+
+@pytest.mark.parametrize("plan", PLANS[:7], ids=str)
+def test_last_slot_decides_nothing_but_the_tiles_run(plan):
+    """A range looks for its last valid slot only where its last slot is masked:
+    rows that end in a valid slot behind masked ones, in an index past the cache,
+    or (paged) in a slot of an unbacked block give the bits of the same row with
+    the masked slots written as -1 and of a call of one query, which looks at none."""
+    K, L, bs = 384, 960, 16
+    q, kv, qr, kr, ids = (t.cuda() for t in _case(3, [K] * 32, K=K, L=L))
+    ids[0, 0, 0, 5:K - 1] = -1           # one valid slot at either end
+    ids[0, 1, 0, 70:] = L                # past the cache
+    ids[0, 2, 0, 33:] = -2 ** 31
+    ids[0, 3, 0, :-2] = -1               # the last but one
+    ids[0, 3, 0, -1] = 2 ** 31 - 1
+    ids[0, 4, 0, K - 40:] = 17           # of an unbacked block, below
+    table = torch.randperm(L // bs, generator=torch.Generator().manual_seed(1)).int().cuda()[None]
+    pool, rpool = torch.empty_like(kv).view(L // bs, bs, 1, 512), torch.empty_like(kr).view(L // bs, bs, 1, 64)
+    pool[table[0].long()], rpool[table[0].long()] = kv.view(L // bs, bs, 1, 512), kr.view(L // bs, bs, 1, 64)
+    table[0, 1] = -1
+    seen = torch.where((ids < 0) | (ids >= L) | (ids // bs == 1), -1, ids)
+    got = dsa_amd.forward(q, pool, qr, rpool, ids, config=plan, block_table=table)
+    want = dsa_amd.forward(q, kv, qr, kr, seen, config=plan)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    for s in range(6):
+        one = dsa_amd.forward(q[:, s:s + 1].contiguous(), kv, qr[:, s:s + 1].contiguous(), kr,
+                              seen[:, s:s + 1].contiguous(), config=plan)
+        for a, b in zip((got[0][:, s:s + 1], got[1][:, :, s:s + 1], got[2][:, :, s:s + 1]), one):
+            assert torch.equal(a, b), s
