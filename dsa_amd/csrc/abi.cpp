@@ -123,13 +123,17 @@ int plan_impl(int B, int SQ, int H, int L, int TOPK, int num_cus, bool fp8, bool
     // prefills.  The specialised-wave variants (32-row tiles, gather waves)
     // measured within ±9 % of the column-split ones, ahead where a workgroup
     // holds 32 heads.  The 64-head ping-pong variant (two tile streams) replaces
-    // wide<2,2> wherever 64-head workgroups pay (4096 queries of 64 heads 1,085
-    // against 1,360 us) and 128-head plans that fill less than half of the CUs
-    // (100 queries of 128 heads 72 against 83 us); it is behind at 8- and
-    // 16-token decodes (25.9 against 21.5 us at 8).  Its and the 128-head
-    // variants' costs were fitted by timing the old and the new choice on 187
-    // shapes whose plan they change (16 to 128 heads, 1 to 4096 tokens): median
-    // 10 % faster, one (20 tokens of 32 heads) 6 % slower.
+    // wide<2,2> for 64-head chunks of more than about 512 slots (4096 queries of
+    // 64 heads, 2048 slots, 1,085 against 1,360 us; at 512 the two costs are
+    // within 1 % and wide<2,2> is taken) and 128-head plans that fill less than
+    // half of the CUs (100 queries of 128 heads 72 against 83 us); it is behind
+    // at 8- and 16-token decodes (25.9 against 21.5 us at 8).  Its and the
+    // 128-head variants' costs were fitted on 187 shapes whose plan they change,
+    // and both choices timed on 333 (16 to 128 heads, 1 to 700 tokens, 256 to
+    // 2048 slots): median 7 % faster; slower remain 32-head decodes that take
+    // xs<2> with twice the splits of xs<1> (20 tokens of 32 heads or 5 of 128,
+    // 2048 slots, 23.4 against 22.6 and 22.0 against 21.2 us) and 32-head chunks
+    // of 256 slots (700 queries 57.2 against 55.5 us).
     struct Variant {
         int hpg, kvw, bn, stages, mfma, pv_cols;
         bool bf16, fp8;
@@ -152,6 +156,11 @@ int plan_impl(int B, int SQ, int H, int L, int TOPK, int num_cus, bool fp8, bool
     constexpr double kClockMHz = 2200.0, kPrologueCycles = 9000.0, kLaunchUs = 2.0;
     constexpr double kHbmBytesPerUs = 4.8e6, kCuBytesPerUs = 3.0e4;                // sustained gather rates
     constexpr double kMergeUs = 2.0, kMergeWgBytesPerUs = 4.2e4, kMergeBytesPerUs = 6.0e6;
+    // The merge folds 16 partials at a time, every load of a batch in flight; a
+    // second batch waits for the first (5 tokens of 32 heads, 1500 slots: 16
+    // splits 15.0 us, 24 splits 16.6 us).
+    constexpr int kMergeBatch = 16;
+    constexpr double kMergeBatchUs = 0.5;
     constexpr double kFp8TileCycles = 1200.0;  // expanding a 64-row fp8 tile to bf16 in LDS
     constexpr double kFusedUs = 0.5, kFusedXsUs = 1.0, kFusedBytesPerUs = 3.0e4;  // in-kernel merge: count-in, one CU's read rate
     const int64_t tokens = (int64_t)B * SQ;
@@ -185,7 +194,7 @@ int plan_impl(int B, int SQ, int H, int L, int TOPK, int num_cus, bool fp8, bool
                 const double merge_wgs = (double)tokens * ((H + 1) / 2);
                 const double bw = merge_wgs * kMergeWgBytesPerUs < kMergeBytesPerUs ? merge_wgs * kMergeWgBytesPerUs
                                                                                     : kMergeBytesPerUs;
-                merge_us = kMergeUs + bytes / bw;
+                merge_us = kMergeUs + bytes / bw + kMergeBatchUs * ((split - 1) / kMergeBatch);
             }
             double cost = kLaunchUs + main_us + merge_us;
             int fused = 0;

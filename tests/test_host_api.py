@@ -178,6 +178,14 @@ def test_prefill_calls_bucket_their_rows_first():
     assert all(l.name != "bucket_rows" for l in launches)
 
 
+@pytest.mark.parametrize("topk", [1500, 1536])
+@pytest.mark.parametrize("tokens,heads", [(1, 128), (3, 48), (5, 32), (8, 16), (10, 16)])
+def test_plans_merge_at_most_one_batch_of_partials(tokens, heads, topk):
+    """The merge folds 16 partials at a time: a small decode does not split
+    further for the sake of one tile less a workgroup."""
+    assert plan_call((tokens, 1, heads, 32768, topk), cores=256)[0].split <= 16
+
+
 def test_plan_call_fused_merge_is_one_launch():
     shape = CASE_SHAPES["c3_decode_h16_mtp"]
     config, partials, launches = plan_call(shape, cores=256)
