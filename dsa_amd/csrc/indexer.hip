@@ -247,8 +247,10 @@ constexpr int kBins0 = 4096;      // first digit: key bits 31..20 (sign, exponen
 constexpr int kCandCap = 1536;    // entries sharing T's upper 16 bits kept in LDS as (s, key)
 constexpr int kStageOut = 4096;   // largest TOPK whose row is assembled in LDS
 
+// REP: copies of each first-digit bin (see topk_registers).
+template <int REP>
 struct TopkShared {
-    uint32_t hist[kBins0];  // digit histograms; rows in registers: afterwards the selected s
+    uint32_t hist[kBins0 * REP];  // digit histograms; rows in registers: afterwards the selected s
     union {
         struct {  // topk_select
             uint32_t cand_s[kCandCap];
@@ -357,7 +359,8 @@ __device__ __forceinline__ void upper4(const Row& row, int s, uint32_t h[4]) {
 //   sweep: the segment counts place every wave's writes.
 // Every pass reads the row from memory (rows longer than kRegKeys); a 16-bit
 // prefix shared by more than kCandCap entries is resolved over the whole row.
-__device__ __forceinline__ void topk_select(TopkShared& sh, const Row& row, int32_t* __restrict__ dst, int n,
+template <int REP>
+__device__ __forceinline__ void topk_select(TopkShared<REP>& sh, const Row& row, int32_t* __restrict__ dst, int n,
                                             int K) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -677,13 +680,22 @@ __device__ __forceinline__ uint32_t waves_below(const uint32_t* v, int wave, int
 // with 32 keys per thread or fewer two workgroups share a CU, one reading or in
 // a barrier while the other counts.  Measured: see launch_indexer_topk.
 // Slots past n hold key 0 and the largest s: n > K, so they are never taken.
+//
+// Long rows count their first digit in four copies of each bin, a lane's by its
+// number, so that logits that share a bin (zeros, ties) meet four times less
+// often: 8 rows of 32768, half of them zeros, 19.4 us instead of 27.7, 128 rows
+// of 65536 30.6 instead of 47.9; without ties 16.6 and 30.8 us either way.
+constexpr int topk_rep(int kpt) { return kpt >= 32 ? 4 : 1; }
 template <int KPT>
-__device__ __forceinline__ void topk_registers(TopkShared& sh, const Row& row, int32_t* __restrict__ dst, int n,
+__device__ __forceinline__ void topk_registers(TopkShared<topk_rep(KPT)>& sh, const Row& row, int32_t* __restrict__ dst, int n,
                                                int K) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int G = 4;  // steps per uniform skip
+    constexpr int REP = topk_rep(KPT);
+    static_assert(REP == 1 || REP == 4, "bin copies");
+    uint32_t* const hist = sh.hist + (lane & (REP - 1));
     // 64-entry steps of a wave, a multiple of G, <= KPT
     const int steps = (n + G * kTopkThreads - 1) / (G * kTopkThreads) * G;
     const int lo = wave * 64 * steps;
@@ -703,7 +715,8 @@ __device__ __forceinline__ void topk_registers(TopkShared& sh, const Row& row, i
     for (int c = 0; c < KPT; ++c) key[c] = 0;
     const int voff = (lo + lane) * 4;
     TOPK_STEPS(c) key[c] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(row.rs, voff + c * 256, 0, 0);
-    reinterpret_cast<uint4*>(sh.hist)[tid] = uint4{0, 0, 0, 0};
+#pragma unroll
+    for (int r = 0; r < REP; ++r) reinterpret_cast<uint4*>(sh.hist)[tid + r * kTopkThreads] = uint4{0, 0, 0, 0};
     static_assert(kBins0 == 4 * kTopkThreads, "four first-digit bins per thread");
     if (tid < 512) reinterpret_cast<uint4*>(sh.hist_low)[tid] = uint4{0, 0, 0, 0};
     __syncthreads();
@@ -713,22 +726,41 @@ __device__ __forceinline__ void topk_registers(TopkShared& sh, const Row& row, i
     if (lo + 64 * steps <= n) {  // every slot holds an entry
         TOPK_STEPS(c) {
             key[c] = float_key(__uint_as_float(key[c]));
-            atomicAdd(&sh.hist[key[c] >> 20], 1u);
+            atomicAdd(&hist[(key[c] >> 20) * REP], 1u);
         }
     } else {
         TOPK_STEPS(c) {
             const bool in = lo + c * 64 + lane < n;
             key[c] = in ? float_key(__uint_as_float(key[c])) : 0u;
-            if (in) atomicAdd(&sh.hist[key[c] >> 20], 1u);
+            if (in) atomicAdd(&hist[(key[c] >> 20) * REP], 1u);
         }
     }
     __syncthreads();
     uint32_t need = (uint32_t)K;  // entries still to take among those matching the digits so far
     {
         // thread tid owns bins kBins0 - 4 - 4 tid .. + 3, counted from the top
-        const uint4 v = *reinterpret_cast<const uint4*>(&sh.hist[kBins0 - 4 - 4 * tid]);
-        const uint32_t c[4] = {v.w, v.z, v.y, v.x};
-        const uint32_t sum = v.x + v.y + v.z + v.w;
+        uint32_t c[4];
+        if constexpr (REP == 1) {
+            const uint4 v = *reinterpret_cast<const uint4*>(&sh.hist[kBins0 - 4 - 4 * tid]);
+            c[0] = v.w, c[1] = v.z, c[2] = v.y, c[3] = v.x;
+        } else {
+            // bin kBins0 - 1 - 4 tid - j: one uint4 of copies, read in an order
+            // that puts 16 lanes on 16 bank groups
+            const uint4* bins = reinterpret_cast<const uint4*>(sh.hist) + (kBins0 - 1 - 4 * tid);
+            const int turn = tid + (tid >> 2);
+            uint32_t s[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint4 v = bins[-((q + turn) & 3)];
+                s[q] = v.x + v.y + v.z + v.w;
+            }
+            uint32_t t[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) t[q] = turn & 1 ? s[(q + 3) & 3] : s[q];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) c[q] = turn & 2 ? t[(q + 2) & 3] : t[q];
+        }
+        const uint32_t sum = c[0] + c[1] + c[2] + c[3];
         const uint32_t incl = wave_incl_scan(sum);
         if (lane == 63) sh.wgt[wave] = incl;
         __syncthreads();
@@ -813,7 +845,7 @@ __device__ __forceinline__ void topk_registers(TopkShared& sh, const Row& row, i
 template <int KPT, bool LONG>
 __global__ __launch_bounds__(kTopkThreads, KPT <= 32 ? 8 : 4) void indexer_topk_kernel(
     const float* __restrict__ logits, const int32_t* __restrict__ len, int32_t* __restrict__ out, int L, int K) {
-    __shared__ __attribute__((aligned(16))) TopkShared sh;
+    __shared__ __attribute__((aligned(16))) TopkShared<topk_rep(KPT)> sh;
     const int r = blockIdx.x;
     const int n = min(max(len[r], 0), L);
     int32_t* dst = out + (int64_t)r * K;

@@ -58,3 +58,16 @@ def test_many_rows_of_every_length():
     logits = torch.randn(1, rows, L, generator=g).abs().sqrt()
     lengths = torch.randint(0, L + 1, (1, rows), generator=g, dtype=torch.int32)
     _check(logits, lengths, 512, "many")
+
+
+@pytest.mark.parametrize("L", [16384, 16385, 20000, 32768])
+@pytest.mark.parametrize("rows", [3, 40])
+def test_rows_of_zeros(L, rows):
+    """Logits that a relu has clipped: half of a row in one first-digit bin, the
+    threshold above it, in it, and among its ties."""
+    g = torch.Generator().manual_seed(L + rows)
+    logits = torch.randn(1, rows, L, generator=g).clamp(min=0)
+    lengths = torch.randint(L // 2, L + 1, (1, rows), generator=g, dtype=torch.int32)
+    lengths[0, 0] = L
+    for k in (64, L // 4, L // 2 + L // 4):
+        _check(logits, lengths, k, (L, rows, k))
