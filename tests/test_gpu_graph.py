@@ -88,6 +88,48 @@ def test_captured_forward_replays_bitwise(shape, config, dv):
             assert torch.equal(a, b), (tag, rep)
 
 
+@pytest.mark.parametrize("shape,L,K,block,dv", [((1, 300, 128), 1024, 512, 0, 0),      # ping-pong, no split
+                                                ((1, 300, 96), 1024, 4096, 0, 128),     # split, merge and projection
+                                                ((2, 130, 16), 96, 64, 16, 0),          # paged
+                                                ((1, 257, 16), 1024, 4096, 0, 0)],      # merged in the kernel
+                         ids=str)
+def test_captured_fp8_chunk_replays_bitwise(shape, L, K, block, dv):
+    """A chunk that expands its fp8 cache first: the expanded rows, the bucketed
+    indices, partials and counters come from the graph's pool, and every replay
+    expands the rows it finds."""
+    B, SQ, H = shape
+    data = _case(SQ + H, B, SQ, H, L=L, K=K)
+    rows = dsa_amd.quantize_kv_fp8(data[1], data[3])
+    table = None
+    if block:
+        table = torch.randperm(B * L // block, generator=torch.Generator().manual_seed(2)).int().cuda().view(B, -1)
+        table[0, 1] = -1
+        rows = rows.view(B * L // block, block, 1, 656)
+    w = (torch.randn(H, dv, 512, generator=torch.Generator().manual_seed(H)) / 23).bfloat16().cuda() if dv else None
+    args = (data[0], rows, data[2], None, data[4])
+    kw = {"block_table": table, "w_uv": w}
+    (_, launches) = dsa_amd.forward(*args, return_kernels=True, **kw)
+    assert launches[0].name == "expand_rows"
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        static_out, captured = dsa_amd.forward(*args, return_kernels=True, **kw)
+    assert captured == launches
+    torch.cuda.synchronize()
+    for rep in range(4):
+        if rep == 2:
+            fresh = _case(SQ + H + 1000, B, SQ, H, L=L, K=K)
+            for i in (0, 2, 4):
+                data[i].copy_(fresh[i])
+            rows.copy_(dsa_amd.quantize_kv_fp8(fresh[1], fresh[3]).view(rows.shape))
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = dsa_amd.forward(*args, **kw)
+        torch.cuda.synchronize()
+        for a, b in zip(static_out, eager):
+            assert torch.equal(a, b), (shape, rep)
+
+
 def test_two_fused_graphs_replayed_out_of_order():
     """Two fused-merge calls captured into two graphs (on torch's shared
     capture stream), then the second graph replayed first and both replayed

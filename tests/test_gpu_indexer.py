@@ -5,8 +5,9 @@ ABI) with the CPU oracle.
   defined entries (s < length); bf16 inputs, FP32 accumulation on both sides;
 * top-k: bit-exact against the oracle given the same logits (integer output),
   including ties, -0.0 / +0.0, -inf, rows shorter than TOPK, empty rows,
-  constant rows, rows whose keys share one first-digit bin (no candidate
-  compaction) and rows longer than the 65536 keys the kernel caches in LDS;
+  constant rows, rows whose keys share one first-digit bin, at lengths on both
+  sides of 32768 (longer ones are split over 8 workgroups where the rows are
+  few) and of 65536 (longer ones are not held in registers);
 * end to end: the selected indices drive dsa_amd.forward, checked against the
   attention oracle on the same indices.
 """
@@ -78,15 +79,28 @@ def test_indexer_logits_parity(tag, seed, B, SQ, HI, L, mode):
 TOPK_CASES = [
     ("ties", 10, 3, 4, 3000, 512, "ties"),
     ("short rows", 11, 2, 3, 600, 2048, None),
-    ("long cached rows", 12, 1, 2, 40000, 2048, None),
-    ("uncached rows", 14, 1, 2, 70000, 2048, None),
+    ("long rows in registers", 12, 1, 2, 40000, 2048, None),
+    ("rows beyond the registers", 14, 1, 2, 70000, 2048, None),
     ("signed zeros and -inf", 13, 1, 2, 5000, 1000, "zeros"),
     ("narrow values", 15, 2, 2, 20000, 2048, "narrow"),
     ("constant rows", 16, 1, 3, 3000, 700, "constant"),
-    # more first-digit candidates than the segmented path keeps in LDS (8192)
     ("constant long rows", 17, 1, 2, 20000, 2048, "constant"),
-    ("32 rows", 18, 8, 4, 9000, 2048, None),      # the most rows the segmented path takes
-    ("64 rows", 19, 16, 4, 5000, 1024, None),     # one workgroup per row either way
+    ("32 rows", 18, 8, 4, 9000, 2048, None),
+    ("64 rows", 19, 16, 4, 5000, 1024, None),
+    # rows above 32768: the segmented kernels, or one workgroup per row
+    ("ties, long", 30, 3, 2, 33000, 512, "ties"),
+    ("signed zeros and -inf, long", 31, 1, 2, 36000, 9000, "zeros"),
+    ("narrow values, long", 32, 2, 2, 40000, 2048, "narrow"),
+    # more first-digit candidates than the segmented path keeps in LDS (8192)
+    ("constant, long", 33, 1, 2, 33001, 2048, "constant"),
+    ("32 long rows", 34, 8, 4, 33000, 2048, None),   # the most rows the segmented path takes
+    ("33 long rows", 35, 11, 3, 33000, 1024, None),  # one workgroup per row either way
+    # above 65536 a row is read from memory once per digit; more than 1536
+    # entries that share T's upper 16 bits are resolved over the whole row
+    ("ties, beyond the registers", 36, 1, 3, 66001, 700, "ties"),
+    ("narrow values, beyond the registers", 37, 1, 2, 70000, 2048, "narrow"),
+    ("constant, beyond the registers", 38, 1, 2, 65537, 2048, "constant"),
+    ("signed zeros and -inf, beyond the registers", 39, 1, 2, 70000, 20000, "zeros"),
 ]
 
 
@@ -104,7 +118,7 @@ def test_indexer_topk_bit_exact(tag, seed, B, SQ, L, K, mode, segmented):
         logits[..., 1::3] = 0.0
         logits[..., 2::7] = -float("inf")
         lengths[:] = L
-    elif mode == "narrow":  # one first-digit bin holds every key: no candidate compaction
+    elif mode == "narrow":  # one first-digit bin holds every key
         logits = 1.0 + logits * 1e-6
     elif mode == "constant":
         logits = torch.full((B, SQ, L), 0.25)

@@ -20,8 +20,12 @@ def _gpu():
 
 
 def _check(logits, lengths, k, tag):
-    got = dsa_amd.indexer_topk(logits.cuda(), lengths.cuda(), k)
-    assert torch.equal(got.cpu(), O.indexer_topk_ref(logits, lengths, k)), tag
+    """Also without the segmented kernels, which few rows above 32768 would take."""
+    want = O.indexer_topk_ref(logits, lengths, k)
+    few_long = logits.shape[0] * logits.shape[1] <= 32 and logits.shape[2] > 32768
+    for segmented in (True, False) if few_long else (True,):
+        got = dsa_amd.indexer_topk(logits.cuda(), lengths.cuda(), k, segmented=segmented)
+        assert torch.equal(got.cpu(), want), (tag, segmented)
 
 
 @pytest.mark.parametrize("L", [2, 63, 64, 65, 4095, 4096, 4097, 8192, 8193, 16384, 16385, 32768, 32769, 65536, 65537])
