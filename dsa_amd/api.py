@@ -192,7 +192,10 @@ def plan_call(shape, config=None, cores: int = 256, kv_fp8: bool = False, w_uv_d
 
     Pure host logic (reference: dsa/api.py:88-113); usable without a GPU.
     ``kv_fp8``: the call reads fp8 kv rows, which only the narrow variants
-    (``mfma=16``) do.  ``w_uv_dim``: the value head dimension of a W_UV
+    (``mfma=16``) do; the plan can be given as ``config``.  A default call of a
+    shape that :func:`expands_rows` names runs the plan of the bf16 call behind
+    an ``expand_rows`` launch instead (``forward(return_kernels=True)`` returns
+    the launches made).  ``w_uv_dim``: the value head dimension of a W_UV
     projection that follows (no reference counterpart): a split plan then
     merges and projects in one launch after the main kernel (its in-kernel
     merge, if any, is not used: the W_UV launch is there anyway), a plan
@@ -554,6 +557,7 @@ def _has_room(size: int, device) -> bool:
 
 
 def _expand_grid(rows: int) -> int:
+    """Workgroups of the expansion (mirrors kv_rows.hip: grid_for, four rows a wave)."""
     return min(-(-rows // 16), 4096)
 
 

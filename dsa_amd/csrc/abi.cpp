@@ -162,7 +162,8 @@ int plan_impl(int B, int SQ, int H, int L, int TOPK, int num_cus, bool fp8, bool
     constexpr int kMergeBatch = 16;
     constexpr double kMergeBatchUs = 0.5;
     constexpr double kFp8TileCycles = 1200.0;  // expanding a 64-row fp8 tile to bf16 in LDS
-    constexpr double kFusedUs = 0.5, kFusedXsUs = 1.0, kFusedBytesPerUs = 3.0e4;  // in-kernel merge: count-in, one CU's read rate
+    // in-kernel merge: count-in (more from the specialised waves), one CU's read rate
+    constexpr double kFusedUs = 0.5, kFusedXsUs = 1.0, kFusedBytesPerUs = 3.0e4;
     const int64_t tokens = (int64_t)B * SQ;
     const double gathered = (double)tokens * TOPK * (fp8 ? 656.0 : 1152.0);
     double best = -1.0, best_wg = 0.0;
@@ -600,7 +601,7 @@ int dsa_indexer_logits(const uint16_t* q_idx, const uint16_t* k_idx, const float
         p.tiles_per_wg = (int)((work * p.ks + 2047) / 2048);
         if (p.tiles_per_wg > p.ntiles) p.tiles_per_wg = p.ntiles;
     } else {
-        constexpr int kCus = 256, kStartStages = 3;
+        constexpr int kCus = 256, kStartStages = 3;  // a whole MI355X: the split has no device to ask
         const int64_t slots = kCus * (p.ks == 4 ? 1 : 2);
         int64_t best = -1;
         for (int64_t rounds = 1; rounds <= 8; ++rounds) {  // the most ranges that fit in so many rounds

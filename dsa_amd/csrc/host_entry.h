@@ -12,8 +12,10 @@ extern "C" {
 // fp8 cache rows (656 bytes, see dsa_fwd_options.kv_format) of `rows` bf16
 // rows: kv [rows, 512] (16-byte aligned), k_rope [rows, 64] (4-byte aligned),
 // out [rows, 656] (16-byte aligned).  pow2 != 0: each 128-wide block's scale
-// is the least power of two >= amax / 448, else amax / 448 itself; a block
-// whose amax is 0 or NaN keeps scale 1.
+// is the least power of two >= amax / 448, else amax / 448, both as tensor code
+// computes them on the GPU: the quotient as a product with the rounded
+// reciprocal, 2^k beyond |k| = 15 as powf gives it (some units in the last
+// place off for some k).  A block whose amax is 0 or NaN keeps scale 1.
 int dsa_kv_quantize_rows(const uint16_t* kv, const uint16_t* k_rope, uint8_t* out, int64_t rows, int pow2,
                          void* stream);
 

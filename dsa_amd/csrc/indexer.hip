@@ -678,7 +678,9 @@ __device__ __forceinline__ uint32_t waves_below(const uint32_t* v, int wave, int
 // (12, 10, 10 bits) of LDS histogram fix T, ballots count and place the output.
 // Bound by instruction issue (about 35 per 64 entries over the five passes);
 // with 32 keys per thread or fewer two workgroups share a CU, one reading or in
-// a barrier while the other counts.  Measured: see launch_indexer_topk.
+// a barrier while the other counts.  With 32 keys the 64 registers this leaves a
+// thread do not hold everything: 14 spill (44 bytes of scratch), 12 or 13 with
+// 64 keys.  Measured: see launch_indexer_topk.
 // Slots past n hold key 0 and the largest s: n > K, so they are never taken.
 //
 // Long rows count their first digit in four copies of each bin, a lane's by its

@@ -2392,7 +2392,8 @@ __global__ __launch_bounds__(64 * XsLds<HB>::WAVES, 1) void sparse_mla_fwd_xs(Fw
 // A group's state covers its own tiles only; the epilogue scales both to the
 // common max and adds them, half of the columns in each group.  Every half
 // gathers a tile (with 128 heads, every other half), so two tiles are in
-// flight.  Measured, 4096 queries of 64 heads over 8192 rows: 1,085 us against
+// flight.  At 256 registers a wave 2 VGPRs and 12 SGPRs spill (12 bytes of
+// scratch), none of them in the tile loop.  Measured, 4096 queries of 64 heads over 8192 rows: 1,085 us against
 // 1,360 us for wide<2,2>; 2 x 3001 queries from position 0, where the
 // compaction drops a third of the slots, 1,146 against 1,990 us.
 constexpr int kPPWaves = 8;
@@ -2428,11 +2429,11 @@ struct PPLds {
     __device__ static uint32_t stage(uint32_t lds, int t) { return lds + (uint32_t)(t % NSTAGE) * STAGE_BYTES; }
 };
 
-
-// Gather of tile t, by the four waves of group 0 (gw = wave 0..3): kv rows
-// 8 gw .. 8 gw + 7 (one instruction per row) and rope rows 8 gw .. 8 gw + 7
-// (one instruction).  Group 1 issues nothing: the gathers are issued in the
-// half-steps in which group 0 runs PV, off the critical QK path.
+// Gather of tile t, by the four waves of one group (gw = 0..3 within it): kv
+// rows 8 gw .. 8 gw + 7 (one instruction per row) and rope rows 8 gw .. 8 gw + 7
+// (one instruction), issued in the half-steps in which that group runs PV, off
+// the critical QK path.  With 128 heads group 0 issues every tile and group 1
+// none; with ALT each group issues the tiles that the other one scores next.
 __device__ __forceinline__ void pp_issue(const FwdParams& p, const Gather& gt, int t, uint32_t stage,
                                          uint32_t idx_lds, int gw, int lane) {
     // Lane-dependent addresses from an opaque copy of the lane id: hoisted out
@@ -2930,10 +2931,12 @@ int fwd_index_cap(int hpg, int bn, int pv_cols) {
 int launch_fwd(const FwdParams& p, int hpg, int kvw, int bn, int stages, int mfma, int pv_cols, hipStream_t stream) {
     if (!fwd_variant_exists(hpg, kvw, bn, stages, mfma, pv_cols)) return (int)hipErrorInvalidValue;
     if (p.kv_fp8 && (mfma != 16 || pv_cols != 512)) return (int)hipErrorInvalidValue;  // fp8 rows: narrow variants only
-    // Chunks of one sequence's queries look for the last valid slot first (the
-    // ping-pong kernels compact in any case); decode calls, whose rows are full
-    // but for a short context, run the kernels without that step (it costs the
-    // 8-token decode 0.3 us of 21).
+    // Chunks of one sequence's queries look for the last valid slot first, in the
+    // 16- and 32-head column-split and specialised-wave kernels and the fp8
+    // narrow ones.  The ping-pong kernels compact their slots in any case; the
+    // wide kernels, the 64-head column-split one and the bf16 narrow ones run
+    // every tile.  Decode calls, whose rows are full but for a short context, run
+    // the kernels without that step (it costs the 8-token decode 0.3 us of 21).
     const bool trim = p.SQ >= kTrimMinQueries;
     if (pv_cols == 128) {
         if (hpg == 128) return launch(sparse_mla_fwd_pp<false>, p, stream, kPPThreads);

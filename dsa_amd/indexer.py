@@ -18,7 +18,9 @@ from . import _lib
 
 INDEX_DIM = 128
 INDEX_HEADS = (32, 64)
-SEGMENTED_MIN_LENGTH = 32768  # rows up to this length take one workgroup (kIndexerSegMinKeys)
+# Rows up to this length take one workgroup (kernels.h: kIndexerSegMinKeys, which
+# decides; here it saves the workspace).
+SEGMENTED_MIN_LENGTH = 32768
 
 
 def _device_ok(device, tensors):

@@ -13,10 +13,15 @@ that value is exact and they expand the rows with one conversion
 instruction per two values.  :func:`quantize_kv_fp8` writes such rows from a
 bf16 cache: per 128-dim block the scale is the smallest power of two with
 ``amax / scale <= 448`` (e4m3 is floating point, so a power-of-two scale
-costs no relative precision), or exactly ``amax / 448`` with
-``pow2_scales=False``.  Tensors on a ROCm GPU are written by one kernel
-(``csrc/kv_rows.hip``), any other call (CPU tensors, traced or transformed
-ones) by the same arithmetic as tensor code, to the same bytes.
+costs no relative precision), or ``amax / 448`` with ``pow2_scales=False``.
+
+Tensors on a ROCm GPU are written by one kernel (``csrc/kv_rows.hip``), any
+other call (CPU tensors, traced or transformed ones, a package whose library is
+not built) by the same arithmetic as tensor code.  The kernel's bytes are those
+of the tensor code on the same GPU.  On the CPU the two differ in the last place
+of some scales: ``amax / 448`` is a product with the rounded reciprocal on the
+GPU, and powers of two beyond 2^15 or below 2^-15 (block maxima above about 10^7
+or below 0.01) are what the GPU's ``powf`` gives.
 """
 from __future__ import annotations
 

@@ -362,7 +362,9 @@ int dsa_indexer_topk(const float* logits, const int32_t* lengths, int32_t* indic
  * leaves most CUs idle; given `workspace` of at least dsa_indexer_topk_ws_bytes bytes
  * (16-byte aligned, any contents), every row is split over 8 workgroups in
  * three launches instead.  Same result bit for bit.  A NULL workspace, or a
- * size query that returns 0 (many rows), selects dsa_indexer_topk's kernel.
+ * size query that returns 0 (many rows), selects dsa_indexer_topk's kernel; so
+ * do rows of up to 32768 keys, for which the size query asks for a workspace
+ * that is then not used.
  */
 int64_t dsa_indexer_topk_ws_bytes(int B, int SQ, int L, int TOPK);
 
