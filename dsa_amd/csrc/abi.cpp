@@ -158,9 +158,10 @@ int plan_impl(int B, int SQ, int H, int L, int TOPK, int num_cus, bool fp8, bool
     constexpr double kMergeUs = 2.0, kMergeWgBytesPerUs = 4.2e4, kMergeBytesPerUs = 6.0e6;
     // The merge folds 16 partials at a time, every load of a batch in flight; a
     // second batch waits for the first (5 tokens of 32 heads, 1500 slots: 16
-    // splits 15.0 us, 24 splits 16.6 us).
+    // splits 15.0 us, 24 splits 16.6 us).  The fp8 variants' costs were fitted
+    // without this.
     constexpr int kMergeBatch = 16;
-    constexpr double kMergeBatchUs = 0.5;
+    const double kMergeBatchUs = fp8 ? 0.0 : 0.5;
     constexpr double kFp8TileCycles = 1200.0;  // expanding a 64-row fp8 tile to bf16 in LDS
     // in-kernel merge: count-in (more from the specialised waves), one CU's read rate
     constexpr double kFusedUs = 0.5, kFusedXsUs = 1.0, kFusedBytesPerUs = 3.0e4;
