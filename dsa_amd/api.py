@@ -425,13 +425,13 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
     output = torch.empty_like(q)
     maximum = torch.empty((batch, 1, queries, heads), device=device, dtype=torch.float32)
     denominator = torch.empty_like(maximum)
-    out_v = None if uv is None else torch.empty((batch, queries, heads, uv[0]), device=device, dtype=torch.bfloat16)
     order = torch.empty_like(indices) if bucket else None
     # The expanded cache after every buffer that the call needs in any case, and
     # given up if the buffers of the plan that reads it do not fit beside it: a
     # call that fits on the fp8 rows never fails for the expansion's sake.
-    expanded = work = None
+    expanded = work = out_v = None
     if fp8 and default_plan and expands_rows(shape):
+        out_v = _uv_output(shape, uv, device)
         bf16 = _call_plan(shape, None, cores, False, uv_dim)
         few = bf16[4] and arrivals is not None and arrivals.numel() < bf16[5]  # counters of the fp8 plan's size
         expanded = None if few else _expanded_cache(kv, block_table, shape)
@@ -497,6 +497,8 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
             rc = lib.dsa_fwd_opts(*args, ctypes.byref(opts), plan, stream)
     if rc:
         _lib.check(rc, "dsa_fwd_main" if merge_uv else "dsa_fwd")
+    if uv is not None and out_v is None:  # beside the main kernel
+        out_v = _uv_output(shape, uv, device)
     if uv is None:
         result = (output, maximum, denominator)
     elif merge_uv:
@@ -513,6 +515,10 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
     if return_kernels:
         return result, launches
     return result
+
+
+def _uv_output(shape, uv, device):
+    return None if uv is None else torch.empty((*shape[:3], uv[0]), device=device, dtype=torch.bfloat16)
 
 
 def _work_buffers(call, arrivals, device, stream):
