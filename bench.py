@@ -635,7 +635,7 @@ class IndexerCall:
         self.largs = [p(q), p(k), p(w), p(lengths), p(self.logits)]
         self.targs = [p(self.logits), p(lengths), p(self.indices)]
         self.lib = _lib.load()
-        # few rows: the segmented selection (8 workgroups per row) over a workspace
+        # few long rows: the segmented selection (8 workgroups per row) over a workspace
         self.ws_bytes = self.lib.dsa_indexer_topk_ws_bytes(q.shape[0], q.shape[1], k.shape[1], topk)
         self.ws = torch.empty(max(self.ws_bytes, 1), device=q.device, dtype=torch.uint8)
 
