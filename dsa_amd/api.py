@@ -413,7 +413,8 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
         cores = _device_cus(device)
     default_plan = config is None
     uv_dim = None if uv is None else uv[0]
-    config, partials, launches, plan, fused, groups = _call_plan(shape, config, cores, fp8, uv_dim)
+    call = _call_plan(shape, config, cores, fp8, uv_dim)
+    config, partials, launches, plan, fused, groups = call
     if fused and arrivals is not None and arrivals.numel() < groups:
         raise ValueError(f"arrivals holds {arrivals.numel()} counters; this call needs {groups}")
     bucket = buckets_rows(shape)
@@ -422,30 +423,26 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
         _register_fast(device, shape, plan, partials)
 
     stream = torch._C._cuda_getCurrentRawStream(device.index)
-    output = torch.empty_like(q)
-    maximum = torch.empty((batch, 1, queries, heads), device=device, dtype=torch.float32)
-    denominator = torch.empty_like(maximum)
-    order = torch.empty_like(indices) if bucket else None
-    # The expanded cache after every buffer that the call needs in any case, and
-    # given up if the buffers of the plan that reads it do not fit beside it: a
-    # call that fits on the fp8 rows never fails for the expansion's sake.
-    expanded = work = out_v = None
+    expanded = out_v = None
     if fp8 and default_plan and expands_rows(shape):
-        out_v = _uv_output(shape, uv, device)
         bf16 = _call_plan(shape, None, cores, False, uv_dim)
         few = bf16[4] and arrivals is not None and arrivals.numel() < bf16[5]  # counters of the fp8 plan's size
-        expanded = None if few else _expanded_cache(kv, block_table, shape)
-        if expanded is not None:
-            try:
-                work = _work_buffers(bf16, arrivals, device, stream)
-            except torch.OutOfMemoryError:
-                expanded = None
-            else:
-                config, partials, launches, plan, fused, groups = bf16
-                launches = (Launch("expand_rows", _expand_grid(batch * length), 256, 0),) + launches
-    if work is None:
-        work = _work_buffers((config, partials, launches, plan, fused, groups), arrivals, device, stream)
-    part_buf, counters = work
+        expanded = None if few else _expanded_cache(kv, block_table, shape, _buffer_bytes(q, indices, uv_dim, bf16))
+    if expanded is not None:
+        # Given up if the call's other buffers do not fit beside it: a call that
+        # fits on the fp8 rows never fails for the expansion's sake.  (It comes
+        # first, so that it finds the block of the last such call whole.)
+        try:
+            buffers = _buffers(q, indices, shape, device, bucket, bf16, arrivals, stream)
+            out_v = _uv_output(shape, uv, device)
+        except torch.OutOfMemoryError:
+            buffers = expanded = out_v = None
+        else:
+            config, partials, launches, plan, fused, groups = bf16
+            launches = (Launch("expand_rows", _expand_grid(batch * length), 256, 0),) + launches
+    if expanded is None:
+        buffers = _buffers(q, indices, shape, device, bucket, call, arrivals, stream)
+    output, maximum, denominator, order, part_buf, counters = buffers
     part_o = part_m = part_l = None
     if part_buf is not None:
         # One buffer carved into part_o, part_m, part_l (each 256-byte aligned):
@@ -521,24 +518,39 @@ def _uv_output(shape, uv, device):
     return None if uv is None else torch.empty((*shape[:3], uv[0]), device=device, dtype=torch.bfloat16)
 
 
-def _work_buffers(call, arrivals, device, stream):
-    """The partials of a split plan and the arrival counters of a fused one,
-    None where the plan (a _call_plan result) needs none."""
-    _, partials, _, _, fused, groups = call
+def _buffers(q, indices, shape, device, bucket, call, arrivals, stream):
+    """The results of a call (a _call_plan result), the bucketed indices, the
+    partials of a split plan and the arrival counters of a fused one; the last
+    three None where the call needs none."""
+    output = torch.empty_like(q)
+    maximum = torch.empty((shape[0], 1, shape[1], shape[2]), device=device, dtype=torch.float32)
+    denominator = torch.empty_like(maximum)
+    order = torch.empty_like(indices) if bucket else None
+    partials = call[1]
     part_buf = None if partials is None else torch.empty(partials[2], device=device, dtype=torch.float32)
-    if not fused:
-        return part_buf, None
-    return part_buf, arrivals if arrivals is not None else _arrival_counters(device, stream, groups)
+    counters = None
+    if call[4]:
+        counters = arrivals if arrivals is not None else _arrival_counters(device, stream, call[5])
+    return output, maximum, denominator, order, part_buf, counters
 
 
-def _expanded_cache(kv, block_table, shape):
+def _buffer_bytes(q, indices, uv_dim, call) -> int:
+    """Bytes of _buffers and _uv_output (counters aside)."""
+    partials = call[1]
+    rows = q.numel() // HEAD_DIM
+    return (2 * q.numel() + 8 * rows + 4 * indices.numel() + (0 if partials is None else 4 * partials[2])
+            + (0 if uv_dim is None else 2 * uv_dim * rows))
+
+
+def _expanded_cache(kv, block_table, shape, others: int):
     """Buffer of the bf16 rows of an fp8 call's logical cache, latent rows then
     rope rows; None where the pool is beyond what a call accepts (the call
-    itself then says so) or the memory is not there (it runs on the fp8 rows)."""
+    itself then says so) or there is no room for it beside the ``others`` bytes
+    that the call needs (it runs on the fp8 rows)."""
     if block_table is not None and kv.shape[0] * kv.shape[1] >= 1 << 25:
         return None
     elems = shape[0] * shape[3] * (HEAD_DIM + ROPE_DIM)
-    if not _has_room(2 * elems, kv.device):
+    if not _has_room(2 * elems + others, kv.device):
         return None
     try:
         return torch.empty(elems, device=kv.device, dtype=torch.bfloat16)
