@@ -403,14 +403,16 @@ __device__ __forceinline__ bool masked_index(const FwdParams& p, int id) {
 // bucketing moves every masked slot there, so a prompt's first tokens, with
 // fewer keys than slots, run the tiles they fill (300 fresh queries of 16 heads
 // with 1024 slots 21 us against 48 us).
-template <int BN>
+template <int BN, int CAP = DSA_IDX_CAP>
 __device__ __forceinline__ int live_tiles(uint32_t idx_lds, int lane, int nt) {
-    for (int i = (nt * BN + 255) / 256 - 1; i >= 0; --i) {
+    int last = 0;
+#pragma unroll
+    for (int i = 0; i < CAP / 256; ++i) {  // every read in flight
         const i32x4 v = lds_load<i32x4>(idx_lds + 1024 * i + 16 * lane);
         const uint64_t b = __ballot(max(max(v[0], v[1]), max(v[2], v[3])) >= 0);
-        if (b) return min(nt, (256 * i + 256 - 4 * __builtin_clzll(b) + BN - 1) / BN);
+        last = b ? 256 * i + 256 - 4 * __builtin_clzll(b) : last;
     }
-    return min(nt, 1);
+    return min(nt, max(1, (last + BN - 1) / BN));
 }
 
 // Compaction of the workgroup's slots (threads 0..255 hold the masked cache
@@ -1664,7 +1666,7 @@ __global__ __launch_bounds__(PROD ? 2 * kThreads : kThreads, 1) void sparse_mla_
         bool overflow = false;
         if (!PROD || producer) issue_tile<R>(p, gt, 0, R::stage(lds, 0), idx_lds, gw, lane);
         if constexpr (TRIM)
-        if (__builtin_expect(tail, 0)) c.nt = live_tiles<kBN>(idx_lds, lane, c.nt);
+        if (__builtin_expect(tail, 0)) c.nt = live_tiles<kBN, X::IDX_CAP>(idx_lds, lane, c.nt);
         wait_vmcnt<0>();  // Q and tile 0
 
         // 8 bytes behind a 32-byte boundary, as in the narrow kernel: 4096 queries of
