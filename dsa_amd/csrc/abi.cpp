@@ -130,10 +130,9 @@ int plan_impl(int B, int SQ, int H, int L, int TOPK, int num_cus, bool fp8, bool
     // at 8- and 16-token decodes (25.9 against 21.5 us at 8).  Its and the
     // 128-head variants' costs were fitted on 187 shapes whose plan they change,
     // and both choices timed on 333 (16 to 128 heads, 1 to 700 tokens, 256 to
-    // 2048 slots): median 7 % faster; slower remain 32-head decodes that take
-    // xs<2> with twice the splits of xs<1> (20 tokens of 32 heads or 5 of 128,
-    // 2048 slots, 23.4 against 22.6 and 22.0 against 21.2 us) and 32-head chunks
-    // of 256 slots (700 queries 57.2 against 55.5 us).
+    // 2048 slots): median 7 % faster; slower remain 10 tokens of 128 heads and 40
+    // of 32 with 1024 slots (xs<2> with twice the splits of xs<1>, 21.7 against
+    // 21.2 us) and 32-head chunks of 256 slots (700 queries 57.2 against 55.5 us).
     struct Variant {
         int hpg, kvw, bn, stages, mfma, pv_cols;
         bool bf16, fp8;
@@ -162,6 +161,11 @@ int plan_impl(int B, int SQ, int H, int L, int TOPK, int num_cus, bool fp8, bool
     // without this.
     constexpr int kMergeBatch = 16;
     const double kMergeBatchUs = fp8 ? 0.0 : 0.5;
+    // 32-head workgroups beyond 8 splits gain nothing from fewer tiles each: the
+    // merge takes it back (20 tokens of 32 heads, 2048 slots of 16384: 8 splits
+    // 22.1 us, 11 splits 23.2 us; the column-split kernel's 6 splits of 16 heads,
+    // which are then taken, 21.7 us).
+    const double kMergeLateUs = fp8 ? 0.0 : 0.1;
     constexpr double kFp8TileCycles = 1200.0;  // expanding a 64-row fp8 tile to bf16 in LDS
     // in-kernel merge: count-in (more from the specialised waves), one CU's read rate
     constexpr double kFusedUs = 0.5, kFusedXsUs = 1.0, kFusedBytesPerUs = 3.0e4;
@@ -198,6 +202,7 @@ int plan_impl(int B, int SQ, int H, int L, int TOPK, int num_cus, bool fp8, bool
                                                                                     : kMergeBytesPerUs;
                 merge_us = kMergeUs + bytes / bw + kMergeBatchUs * ((split - 1) / kMergeBatch);
             }
+            if (split > 8 && v.hpg == 32) merge_us += kMergeLateUs * (split - 8);
             double cost = kLaunchUs + main_us + merge_us;
             int fused = 0;
             if (fuse && split > 1 && split <= kMaxFusedSplit && v.mfma == 16 && !(v.pv_cols == 128 && v.hpg != 16)) {

@@ -186,6 +186,12 @@ def test_plans_merge_at_most_one_batch_of_partials(tokens, heads, topk):
     assert plan_call((tokens, 1, heads, 32768, topk), cores=256)[0].split <= 16
 
 
+@pytest.mark.parametrize("tokens,heads", [(20, 32), (10, 64), (7, 96), (5, 128)])
+def test_plans_do_not_split_32_heads_for_the_merge(tokens, heads):
+    config = plan_call((tokens, 1, heads, 32768, 2048), cores=256)[0]
+    assert config.split <= 8
+
+
 def test_plan_call_fused_merge_is_one_launch():
     shape = CASE_SHAPES["c3_decode_h16_mtp"]
     config, partials, launches = plan_call(shape, cores=256)
