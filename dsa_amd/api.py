@@ -428,21 +428,32 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
         bf16 = _call_plan(shape, None, cores, False, uv_dim)
         few = bf16[4] and arrivals is not None and arrivals.numel() < bf16[5]  # counters of the fp8 plan's size
         expanded = None if few else _expanded_cache(kv, block_table, shape, _buffer_bytes(q, indices, uv_dim, bf16))
-    if expanded is not None:
-        # Given up if the call's other buffers do not fit beside it: a call that
-        # fits on the fp8 rows never fails for the expansion's sake.  (It comes
-        # first, so that it finds the block of the last such call whole.)
-        try:
-            buffers = _buffers(q, indices, shape, device, bucket, bf16, arrivals, stream)
-            out_v = _uv_output(shape, uv, device)
-        except torch.OutOfMemoryError:
-            buffers = expanded = out_v = None
-        else:
+        if expanded is not None:
             config, partials, launches, plan, fused, groups = bf16
-            launches = (Launch("expand_rows", _expand_grid(batch * length), 256, 0),) + launches
-    if expanded is None:
-        buffers = _buffers(q, indices, shape, device, bucket, call, arrivals, stream)
-    output, maximum, denominator, order, part_buf, counters = buffers
+    while True:
+        try:
+            output = torch.empty_like(q)
+            maximum = torch.empty((batch, 1, queries, heads), device=device, dtype=torch.float32)
+            denominator = torch.empty_like(maximum)
+            order = torch.empty_like(indices) if bucket else None
+            part_buf = None if partials is None else torch.empty(partials[2], device=device, dtype=torch.float32)
+            counters = arrivals if fused else None
+            if fused and counters is None:
+                counters = _arrival_counters(device, stream, groups)
+            if expanded is not None and uv is not None:
+                out_v = _uv_output(shape, uv, device)
+            break
+        except torch.OutOfMemoryError:
+            if expanded is None:
+                raise
+            # The expansion is given up if the call's other buffers do not fit
+            # beside it: a call that fits on the fp8 rows never fails for its
+            # sake.  (It comes first, so that it finds the block of the last
+            # such call whole.)
+            expanded = output = maximum = denominator = order = part_buf = counters = out_v = None
+            config, partials, launches, plan, fused, groups = call
+    if expanded is not None:
+        launches = (Launch("expand_rows", _expand_grid(batch * length), 256, 0),) + launches
     part_o = part_m = part_l = None
     if part_buf is not None:
         # One buffer carved into part_o, part_m, part_l (each 256-byte aligned):
@@ -515,27 +526,12 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
 
 
 def _uv_output(shape, uv, device):
-    return None if uv is None else torch.empty((*shape[:3], uv[0]), device=device, dtype=torch.bfloat16)
-
-
-def _buffers(q, indices, shape, device, bucket, call, arrivals, stream):
-    """The results of a call (a _call_plan result), the bucketed indices, the
-    partials of a split plan and the arrival counters of a fused one; the last
-    three None where the call needs none."""
-    output = torch.empty_like(q)
-    maximum = torch.empty((shape[0], 1, shape[1], shape[2]), device=device, dtype=torch.float32)
-    denominator = torch.empty_like(maximum)
-    order = torch.empty_like(indices) if bucket else None
-    partials = call[1]
-    part_buf = None if partials is None else torch.empty(partials[2], device=device, dtype=torch.float32)
-    counters = None
-    if call[4]:
-        counters = arrivals if arrivals is not None else _arrival_counters(device, stream, call[5])
-    return output, maximum, denominator, order, part_buf, counters
+    return torch.empty((*shape[:3], uv[0]), device=device, dtype=torch.bfloat16)
 
 
 def _buffer_bytes(q, indices, uv_dim, call) -> int:
-    """Bytes of _buffers and _uv_output (counters aside)."""
+    """Bytes of the buffers a call (a _call_plan result) allocates beside an
+    expanded cache (arrival counters aside)."""
     partials = call[1]
     rows = q.numel() // HEAD_DIM
     return (2 * q.numel() + 8 * rows + 4 * indices.numel() + (0 if partials is None else 4 * partials[2])

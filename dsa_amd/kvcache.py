@@ -61,21 +61,23 @@ def quantize_kv_fp8(kv, k_rope, pow2_scales: bool = True):
 
 def _plain_gpu_pair(kv, k_rope):
     """Whether the kernel may read these two tensors: ordinary eager tensors
-    of one ROCm GPU (no subclass, tracing, function or dispatch mode or functorch level
-    between the caller and the storage) with at least one row, and the library
-    built (the rows can be written without it, unlike the attention's results)."""
-    return (_lib.built() and type(kv) is torch.Tensor and type(k_rope) is torch.Tensor and kv.is_cuda and kv.device == k_rope.device
-            and torch.version.hip is not None and kv.numel() > 0 and not torch.compiler.is_compiling()
-            and not torch.jit.is_tracing() and not torch._C._are_functorch_transforms_active()
-            and torch._C._len_torch_dispatch_stack() == 0 and not _function_modes() and not (kv.is_neg() or k_rope.is_neg()))
+    of one ROCm GPU (no subclass, tracing, function or dispatch mode or
+    functorch level between the caller and the storage) with at least one row,
+    and the library built (the rows can be written without it, unlike the
+    attention's results)."""
+    return ((_lib._lib is not None or _lib.built()) and type(kv) is torch.Tensor and type(k_rope) is torch.Tensor
+            and kv.is_cuda and kv.device == k_rope.device and torch.version.hip is not None and kv.numel() > 0
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not torch._C._are_functorch_transforms_active() and torch._C._len_torch_dispatch_stack() == 0
+            and (torch._C._len_torch_function_stack() == 0 or _only_default_devices())
+            and not (kv.is_neg() or k_rope.is_neg()))
 
 
-def _function_modes() -> bool:
-    """Whether a torch_function mode watches the operations.  A default device
-    (``torch.set_default_device``) is such a mode too, but only places tensors
-    that name no device."""
-    return (torch._C._len_torch_function_stack() > 0
-            and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
+def _only_default_devices() -> bool:
+    """Whether the torch_function modes are default devices
+    (``torch.set_default_device``), which only place tensors that name no
+    device: any other mode watches the operations."""
+    return all(type(m) is DeviceContext for m in _get_current_function_mode_stack())
 
 
 def _quantize_gpu(kv, k_rope, lead, pow2_scales):
