@@ -418,8 +418,8 @@ def forward(q, kv, q_rope, k_rope, indices, *, config=None, cores=None, return_k
     if fused and arrivals is not None and arrivals.numel() < groups:
         raise ValueError(f"arrivals holds {arrivals.numel()} counters; this call needs {groups}")
     bucket = buckets_rows(shape)
-    if (default_plan and cores == _device_cus(device) and not fused and not fp8 and scale is None
-            and block_table is None and uv is None and not bucket):
+    if (default_plan and not fused and not fp8 and scale is None and block_table is None and uv is None
+            and not bucket and cores == _device_cus(device)):
         _register_fast(device, shape, plan, partials)
 
     stream = torch._C._cuda_getCurrentRawStream(device.index)
